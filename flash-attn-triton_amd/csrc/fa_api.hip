@@ -171,6 +171,17 @@ hipError_t fa_launch_combine(int dtype, const float* o_part, const float* lse_pa
 
 namespace {
 
+// Merge of the splits of a KV-cache launch that ran on prefill_pp_kernel.
+hipError_t launch_cache_combine(int dtype, const fa::FwdParams& p, int head_dim, hipStream_t st) {
+  const int64_t threads = (int64_t)p.batch * p.seqlen_q * p.heads_q * (head_dim / 4);
+  const int64_t blocks = (threads + 255) / 256;
+  if (blocks > 0x7fffffff) return hipErrorInvalidConfiguration;
+  auto kern = dtype == FA_DTYPE_F16 ? fa::cache_combine_kernel<fa::F16>
+                                    : fa::cache_combine_kernel<fa::BF16>;
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), 0, st, p, head_dim);
+  return hipGetLastError();
+}
+
 // Shared part of fa_bwd_dense / fa_bwd_varlen: checks, scale fields, launch.
 int bwd_launch(const char* name, fa::BwdParams& p, int dtype, int64_t head_dim,
                float softmax_scale, float softcap, const float* alibi_slopes,
@@ -588,10 +599,13 @@ int fa_kvcache_run(const char* name, const void* q, const void* k_cache, const v
     p.o_part = static_cast<float*>(workspace);
     p.lse_part = reinterpret_cast<float*>(static_cast<char*>(workspace) + plan.o_part_bytes);
   }
-  p.heavy_first = 0;
+  p.cache_pp = !f32 && fa::cache_pp_route(p, (int)head_dim, needs_generic(p));
+  p.heavy_first = p.cache_pp && p.causal;
   hipError_t e = launch_fwd(dtype, p, fa::kModeKvcache, (int)head_dim, needs_generic(p),
                             (hipStream_t)stream);
-  if (e == hipSuccess && p.num_splits > 1)
+  if (e == hipSuccess && p.num_splits > 1 && p.cache_pp)
+    e = launch_cache_combine(dtype, p, (int)head_dim, (hipStream_t)stream);
+  else if (e == hipSuccess && p.num_splits > 1)
     e = fa_launch_combine(dtype, p.o_part, p.lse_part, out, lse, plan.num_splits, (int)batch,
                           (int)seqlen_q, (int)heads_q, (int)head_dim, o_stride, lse_stride,
                           (hipStream_t)stream);

@@ -82,6 +82,11 @@ struct FwdParams {
   // the GQA group size (set by the persistent launchers).
   int persist_rounds;
   FastDiv fd_blk, fd_heads, fd_group;
+  // KV-cache launches of prefill_pp_kernel (cache_pp set by the C ABI, which
+  // then merges with cache_combine_kernel; fd_group as above) and paged ones
+  // (division by page_size).
+  int cache_pp;
+  FastDiv fd_page;
   // Dropout of the probabilities (prefill, GENERIC instantiations only).
   DropoutCfg drop;
 };

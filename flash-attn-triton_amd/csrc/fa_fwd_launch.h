@@ -60,15 +60,21 @@ hipError_t launch_prefill_cfg(FwdParams p, hipStream_t st) {
   return hipGetLastError();
 }
 
-// Ping-pong prefill (fa_prefill_pp.h): 8 waves, 256 query rows per workgroup.
-template <class T, int D, bool VARLEN>
+// Ping-pong prefill (fa_prefill_pp.h): 8 waves, 256 rows per workgroup.
+template <class T, int D, int MODE, bool PAGED>
 hipError_t launch_prefill_pp(FwdParams p, hipStream_t st) {
   using Tile = PingPongTile<D>;
-  auto kern = prefill_pp_kernel<T, D, VARLEN>;
+  auto kern = prefill_pp_kernel<T, D, MODE, PAGED>;
   static std::atomic<uint64_t> lds_devices{0};
   if (hipError_t e = set_lds_limit(lds_devices, kern, Tile::LDS_BYTES); e != hipSuccess) return e;
-  p.n_mblocks = (p.seqlen_q + Tile::BM - 1) / Tile::BM;
-  const int64_t total = (int64_t)p.n_mblocks * p.heads_q * p.batch;
+  const int rows = MODE == kPpCache ? p.seqlen_q * p.group : p.seqlen_q;
+  p.n_mblocks = (rows + Tile::BM - 1) / Tile::BM;
+  int64_t total = (int64_t)p.n_mblocks * p.heads_q * p.batch;
+  if (MODE == kPpCache) {
+    total = (int64_t)p.n_mblocks * p.heads_k * p.batch * p.num_splits;
+    p.fd_group = make_fastdiv((uint32_t)p.group);
+  }
+  if (PAGED) p.fd_page = make_fastdiv((uint32_t)p.page_size);
   if (total <= 0) return hipSuccess;
   if (total > 0x7fffffff) return hipErrorInvalidConfiguration;
   p.total_blocks = (int)total;
@@ -121,6 +127,25 @@ hipError_t launch_prefill_persist(FwdParams p, hipStream_t st, bool* launched) {
   return hipGetLastError();
 }
 
+// Paged keys the ping-pong kernel's 8-row tile loads can take.
+inline bool pp_pages(const FwdParams& p) { return p.block_table != nullptr && p.page_size % 8 == 0; }
+
+// KV-cache launches that run on the ping-pong kernel instead of fwd_kernel:
+// head dim 128, more rows than the decode kernel's 32, pages of whole 8-row
+// groups, strides whose 32-row offsets stay far inside 32 bits, and neither
+// ALiBi nor a scale <= 0 (`generic`).  Ahead over the whole of that range:
+// per call with fwd_kernel and with it, bf16, MI355X, 512 queries and 32 / 8
+// heads 614 -> 168 us; 33 rows per KV head (the fewest; 32 KV heads, B8) 515 ->
+// 192 us; 64 queries (B4) 135 -> 102 us, where the host's argument checks bound
+// both.
+inline bool cache_pp_route(const FwdParams& p, int head_dim, bool generic) {
+  constexpr int64_t kMaxStride = (int64_t)1 << 24;   // elements
+  const int64_t rows = (int64_t)p.seqlen_q * p.group;
+  return head_dim == 128 && !generic && rows > 32 && (p.block_table == nullptr || pp_pages(p)) &&
+         p.q_ss <= kMaxStride && p.q_sh * p.group <= kMaxStride && p.k_ss <= kMaxStride &&
+         p.v_ss <= kMaxStride;
+}
+
 template <class T, int D, bool GEN>
 hipError_t launch_prefill(const FwdParams& p, hipStream_t st) {
   if constexpr (GEN) {
@@ -139,11 +164,11 @@ hipError_t launch_prefill(const FwdParams& p, hipStream_t st) {
     // of the block's window for all rows, and the softmax phase outgrows the
     // GEMM phase).
     if constexpr (!GEN) {
-      if (p.cu_q != nullptr) return launch_prefill_pp<T, D, true>(p, st);
+      if (p.cu_q != nullptr) return launch_prefill_pp<T, D, kPpVarlen, false>(p, st);
       bool launched = false;
       hipError_t e = launch_prefill_persist<T, D>(p, st, &launched);
       if (e != hipSuccess || launched) return e;
-      return launch_prefill_pp<T, D, false>(p, st);
+      return launch_prefill_pp<T, D, kPpDense, false>(p, st);
     }
     // The generic epilogue (varlen, ALiBi, softcap, window) does not fit the
     // 168-VGPR budget of 3 waves per SIMD without spilling: 2 waves, in
@@ -170,8 +195,12 @@ hipError_t launch_prefill(const FwdParams& p, hipStream_t st) {
 template <class T, int D, int MODE, bool GEN>
 hipError_t launch_fwd_d(const FwdParams& p, hipStream_t st) {
   if (MODE == kModePrefill) {
-    // Paged varlen keys need a page lookup per key: the general kernel.
+    // Paged varlen keys: a page lookup per 8 keys on the ping-pong kernel, or
+    // per key on the general one.
     if (p.block_table != nullptr) {
+      if constexpr (D == 128 && !GEN) {
+        if (pp_pages(p)) return launch_prefill_pp<T, D, kPpVarlen, true>(p, st);
+      }
       using C = PrefillCfg<D>;
       return launch_fwd_cfg<T, D, C::NW, C::BN, MODE, GEN>(p, p.seqlen_q, p.heads_q * p.batch, st);
     }
@@ -181,6 +210,11 @@ hipError_t launch_fwd_d(const FwdParams& p, hipStream_t st) {
       using C = PrefillCfg<D>;
       return launch_fwd_cfg<T, D, C::NW, C::BN, MODE, GEN>(p, p.seqlen_q, p.heads_q * p.batch, st);
     }
+  }
+  if constexpr (D == 128 && !GEN) {
+    if (p.cache_pp)
+      return p.block_table != nullptr ? launch_prefill_pp<T, D, kPpCache, true>(p, st)
+                                      : launch_prefill_pp<T, D, kPpCache, false>(p, st);
   }
   const int rows = p.seqlen_q * p.group;
   const int outer = p.heads_k * p.batch * p.num_splits;

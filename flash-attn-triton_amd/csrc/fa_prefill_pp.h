@@ -1,5 +1,5 @@
 // Ping-pong FlashAttention-2 prefill forward for gfx950 at head dim 128,
-// fp16 / bf16 (dense, cross and varlen).
+// fp16 / bf16 (dense, cross, varlen, and chunks of queries against a KV cache).
 //
 // Semantics are those of prefill_kernel (fa_prefill_kernel.h), i.e. the
 // reference's dense and varlen forward kernels
@@ -34,6 +34,25 @@
 // c ^ 4 (r & 3) for V, so the K reads of the S^T product (16 rows, one chunk
 // column per 16 lanes) and the V^T transpose reads (ds_read_b64_tr_b16, 4 rows
 // x 4 chunks per 32 lanes) touch distinct bank groups.
+//
+// Paged K/V (varlen with a block table, and the paged cache): the 8 rows a
+// wave copies of every tile lie in one page (page_size % 8 == 0), so a tile
+// load costs the wave one block-table entry, read through the scalar cache
+// one tile ahead and shared by K and V, and the loads stay whole-row DMA.
+//
+// KV-cache mode (kPpCache): the rows of a workgroup are (query, head) pairs of
+// one KV head, head fastest, so the query heads of a group share every K/V
+// tile, and the keys of a sequence are split into ranges of split_tiles tiles
+// (cache_combine_kernel merges them; a sequence that fits one range is written
+// directly).  These forms keep fwd_kernel's precision, which they replaced:
+// unpre-scaled Q, row sums over the fp32 P, and the running max raised with
+// every larger score (slack 0): the largest P of a row is then exactly 1,
+// where a stale max rounds it (measured 2.25e-3 against 2.34e-3 relative error
+// to float64 in bf16, for 5 % of the time).  What bounds them is the
+// GEMM / softmax phase pair, as in the dense form.  Measured on one MI355X,
+// causal, bf16, Hq32 Hk8, page 256: 512 queries against 4 caches of 512 to
+// 8192 keys 584 + 16 us (fwd_kernel + combine) -> 147 + 12 us; 4 full
+// caches of 8192 keys 796 -> 342 us per call.
 #pragma once
 
 #include <type_traits>
@@ -70,9 +89,58 @@ __device__ inline void pp_barrier() {
   __builtin_amdgcn_sched_barrier(0);
 }
 
-// VARLEN: cu_seqlens addressing (an instantiation of its own, so that the
-// dense kernel carries none of its work-item code).
-template <class T, int D, bool VARLEN>
+// The launch forms, instantiations of their own so that the dense kernel
+// carries none of the others' work-item code: dense / cross, cu_seqlens
+// addressing, and a few queries per sequence against a KV cache.
+enum { kPpDense = 0, kPpVarlen = 1, kPpCache = 2 };
+
+// Work item of a KV-cache launch: row block mb, key split and KV group
+// c = b * heads_k + kvh.  Row blocks vary fastest (the blocks of a KV head
+// share its tiles in one L2), the split slowest, so that every sequence's
+// full leading splits go out before the short or empty trailing ones.  KV
+// groups are dealt round-robin over the 8 XCDs; with 1, 2 or 4 groups each
+// takes 8 / n_kv XCDs.
+__device__ inline void work_item_cache(int L, int total, int n_mblocks, int n_kv, int& mb,
+                                       int& split, int& c) {
+  constexpr int kXcds = 8;
+  int k = L;
+  if (n_kv % kXcds == 0) {
+    const int per = n_kv / kXcds;
+    k = L / kXcds;
+    mb = k % n_mblocks;
+    k /= n_mblocks;
+    c = (k % per) * kXcds + L % kXcds;
+    split = k / per;
+  } else if (kXcds % n_kv == 0 && total % kXcds == 0) {
+    c = (L % kXcds) % n_kv;
+    k = (L / kXcds) * (kXcds / n_kv) + (L % kXcds) / n_kv;
+    mb = k % n_mblocks;
+    split = k / n_mblocks;
+  } else {
+    mb = k % n_mblocks;
+    k /= n_mblocks;
+    c = k % n_kv;
+    split = k / n_kv;
+  }
+}
+
+// Visible keys of sequence b of a KV-cache call, clamped to what the cache and
+// the block table hold whatever the device arrays contain; *row is the batched
+// cache's row and *pad its left padding.
+__device__ inline int cache_keys(const FwdParams& p, int b, int* row, int* pad) {
+  int L = p.seqlens_k != nullptr ? p.seqlens_k[b] : p.seqlen_k;
+  int lp = 0;
+  *row = b;
+  if (p.block_table == nullptr) {
+    if (p.cache_rows != nullptr) *row = p.cache_rows[b];
+    if (p.leftpad != nullptr) lp = max(0, min(p.leftpad[b], p.seqlen_k));
+    if (*row < 0 || *row >= p.cache_blocks) L = 0;
+  }
+  *pad = lp;
+  return max(0, min(L, p.seqlen_k - lp));
+}
+
+template <class T, int D, int MODE, bool PAGED>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void prefill_pp_kernel(const FwdParams p) {
   using Tile = PingPongTile<D>;
@@ -87,6 +155,10 @@ void prefill_pp_kernel(const FwdParams p) {
   constexpr int NDB = D / 32;      // 32-dim blocks of O^T
   constexpr int NKB = BN / 32;     // 32-key blocks per tile
   constexpr int NCC = BN / 16;     // 16-key k-steps of O^T
+  constexpr bool VARLEN = MODE == kPpVarlen;
+  constexpr bool CACHE = MODE == kPpCache;
+  static_assert(!PAGED || MODE != kPpDense, "dense K/V are not paged");
+  static_assert(!PAGED || RPI * IPW == 8, "a wave's rows of a tile must be 8 consecutive keys");
 
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem_pp[];
 
@@ -102,17 +174,33 @@ void prefill_pp_kernel(const FwdParams p) {
   // ------------------------------------------------------------ work item
   // Varlen: K/V heads round-robin over the XCDs (ragged sequences load
   // contiguous group ranges unevenly).
-  int mb, id;
-  if (!VARLEN ||
-      !work_item_kv_rr(blockIdx.x, p.total_blocks, p.n_mblocks, p.group, p.heavy_first != 0, mb, id))
-    work_item(blockIdx.x, p.total_blocks, p.n_mblocks, p.heavy_first != 0, kCausalSpan, mb, id);
-  const int hh = id % p.heads_q;
-  const int b = id / p.heads_q;
-  const int kvh = hh / p.group;
+  int mb, hh, b, kvh, split = 0;
+  if constexpr (CACHE) {
+    int c;
+    work_item_cache(blockIdx.x, p.total_blocks, p.n_mblocks, p.batch * p.heads_k, mb, split, c);
+    if (p.heavy_first) mb = p.n_mblocks - 1 - mb;
+    b = c / p.heads_k;
+    kvh = c % p.heads_k;
+    hh = kvh * p.group;   // first query head of the group
+  } else {
+    int id;
+    if (!VARLEN ||
+        !work_item_kv_rr(blockIdx.x, p.total_blocks, p.n_mblocks, p.group, p.heavy_first != 0, mb, id))
+      work_item(blockIdx.x, p.total_blocks, p.n_mblocks, p.heavy_first != 0, kCausalSpan, mb, id);
+    hh = id % p.heads_q;
+    b = id / p.heads_q;
+    kvh = hh / p.group;
+  }
 
-  int Sq, Sk;
-  int64_t q_base, o_base, lse_base, k_base, v_base;
-  if (p.cu_q != nullptr) {
+  int Sq, Sk, qoff32 = (int)p.q_offset;
+  int64_t q_base, o_base, lse_base, k_base = 0, v_base = 0;
+  // Block table of this sequence, in the constant address space: its entries
+  // are wave-uniform and go through the scalar cache, off the vector-memory
+  // counter the tile loads are waited on with.
+  typedef const __attribute__((address_space(4))) int* table_ptr;
+  table_ptr bt_row = nullptr;
+  if constexpr (PAGED) bt_row = (table_ptr)(p.block_table + (int64_t)b * p.bt_stride);
+  if constexpr (VARLEN) {
     const int qs = p.cu_q[b], ks = p.cu_k[b];
     Sq = p.cu_q[b + 1] - qs;
     Sk = p.cu_k[b + 1] - ks;
@@ -122,16 +210,30 @@ void prefill_pp_kernel(const FwdParams p) {
     q_base = (int64_t)qs * p.q_ss;
     o_base = (int64_t)os * p.o_ss;
     lse_base = (int64_t)os * p.lse_ss;
-    k_base = (int64_t)ks * p.k_ss;
-    v_base = (int64_t)ks * p.v_ss;
+    if constexpr (PAGED) {
+      if (p.bt_cols > 0) Sk = (int)min((int64_t)Sk, (int64_t)p.bt_cols * p.page_size);
+    } else {
+      k_base = (int64_t)ks * p.k_ss;
+      v_base = (int64_t)ks * p.v_ss;
+    }
   } else {
     Sq = p.seqlen_q;
     Sk = p.seqlen_k;
     q_base = (int64_t)b * p.q_sb;
     o_base = (int64_t)b * p.o_sb;
     lse_base = (int64_t)b * p.lse_sb;
-    k_base = (int64_t)b * p.k_sb;
-    v_base = (int64_t)b * p.v_sb;
+    if constexpr (CACHE) {
+      int row, lp;
+      Sk = cache_keys(p, b, &row, &lp);
+      if (p.kv_causal_offset) qoff32 = Sk - Sq;
+      if constexpr (!PAGED) {
+        k_base = (int64_t)row * p.k_sb + (int64_t)lp * p.k_ss;
+        v_base = (int64_t)row * p.v_sb + (int64_t)lp * p.v_ss;
+      }
+    } else {
+      k_base = (int64_t)b * p.k_sb;
+      v_base = (int64_t)b * p.v_sb;
+    }
   }
   q_base += (int64_t)hh * p.q_sh;
   o_base += (int64_t)hh * p.o_sh;
@@ -139,18 +241,30 @@ void prefill_pp_kernel(const FwdParams p) {
   k_base += (int64_t)kvh * p.k_sh;
   v_base += (int64_t)kvh * p.v_sh;
 
+  // Rows: query rows of one head, or (cache) the group's heads of query
+  // gr / group as rows gr = query * group + head.
+  const int rows = CACHE ? Sq * p.group : Sq;
+  auto row_query = [&](int gr) __attribute__((always_inline)) {
+    return CACHE ? (int)fdiv((uint32_t)gr, p.fd_group) : gr;
+  };
+  auto row_head = [&](int gr) __attribute__((always_inline)) {
+    return CACHE ? (int)fmod((uint32_t)gr, p.fd_group) : 0;
+  };
+  // Splits that hold no keys write nothing (the combine skips them); split 0
+  // always runs, so that an empty sequence still gets its rows.
+  if (CACHE && split > 0 && (int64_t)split * p.split_tiles * BN >= Sk) return;
+
   const int row0 = mb * BM;
-  if (row0 >= Sq) return;   // whole workgroup: varlen blocks past this sequence
-  const int row_last = min(row0 + BM, Sq) - 1;
+  if (row0 >= rows) return;   // whole workgroup: varlen blocks past this sequence
+  const int row_last = min(row0 + BM, rows) - 1;
 
   const int wrow0 = row0 + 32 * rb;
-  const int qi = wrow0 + c32;
-  const bool row_valid = qi < Sq;
+  const int qi = wrow0 + c32;   // this lane's row
+  const bool row_valid = qi < rows;
   // Positions fit in 32 bits (the host keeps lengths and offsets below 2^29).
-  const int qoff32 = (int)p.q_offset;
-  const int qpos = qi + qoff32;
-  const int qpos_w_min = wrow0 + qoff32;
-  const int qpos_w_max = min(wrow0 + 31, row_last) + qoff32;
+  const int qpos = row_query(qi) + qoff32;
+  const int qpos_w_min = row_query(wrow0) + qoff32;
+  const int qpos_w_max = row_query(min(wrow0 + 31, row_last)) + qoff32;
 
   const int wl = p.window_left, wr = p.window_right;
   const bool causal = p.causal != 0;
@@ -162,12 +276,16 @@ void prefill_pp_kernel(const FwdParams p) {
 
   // Key tiles [t_begin, t_end) any row of the workgroup can see.
   int k_hi = Sk;
-  if (causal) k_hi = min(k_hi, row_last + qoff32 + 1);
-  if (wr >= 0) k_hi = min(k_hi, row_last + qoff32 + wr + 1);
+  if (causal) k_hi = min(k_hi, row_query(row_last) + qoff32 + 1);
+  if (wr >= 0) k_hi = min(k_hi, row_query(row_last) + qoff32 + wr + 1);
   int k_lo = 0;
-  if (wl >= 0) k_lo = max(0, row0 + qoff32 - wl);
-  const int t_begin = k_lo / BN;
-  const int t_end = k_hi > k_lo ? (k_hi + BN - 1) / BN : t_begin;
+  if (wl >= 0) k_lo = max(0, row_query(row0) + qoff32 - wl);
+  int t_begin = k_lo / BN;
+  int t_end = k_hi > k_lo ? (k_hi + BN - 1) / BN : t_begin;
+  if constexpr (CACHE) {   // this split's tiles
+    t_begin = max(t_begin, split * p.split_tiles);
+    t_end = max(t_begin, min(t_end, (split + 1) * p.split_tiles));
+  }
   const int J = t_end - t_begin;
 
   // ------------------------------------------------------------ Q^T in VGPRs
@@ -175,8 +293,11 @@ void prefill_pp_kernel(const FwdParams p) {
   // reference's forward kernel does (attention_kernel.py:492-495), so the
   // scores come out of the MFMAs in log2 units.  bf16 keeps Q as given (its
   // 8-bit mantissa would move the log-sum-exp by ~1.5e-3) and scales every
-  // score in the softmax.
-  constexpr bool kPre = std::is_same<T, F16>::value;
+  // score in the softmax; so do the KV-cache and paged forms, whose callers
+  // have always had the unrounded Q.
+  constexpr bool kPre = std::is_same<T, F16>::value && !CACHE && !PAGED;
+  constexpr float kSlack = CACHE || PAGED ? 0.f : kRescaleSlack;
+  constexpr bool kSumRounded = T::kSumRounded && !CACHE && !PAGED;
   const uint16_t* qg = static_cast<const uint16_t*>(p.q);
   u32x4 qreg[NKC];
   // This wave's 32 Q rows are staged through LDS with whole-row DMA (rows past
@@ -185,9 +306,25 @@ void prefill_pp_kernel(const FwdParams p) {
   // area past the rings.
   static_assert(D == 128, "Q staging holds 256-byte rows");
   uint8_t* const q_st = smem_pp + (grp == 0 ? NS * TILEB + 2 * TILEB : Tile::STAGE_OFF) + sid * 8192;
-  stage_rows_load(make_rsrc_words(qg + q_base + (int64_t)wrow0 * p.q_ss,
-                                  rows_extent(wrow0, Sq, p.q_ss, D)),
-                  lds_address(q_st), (uint32_t)(p.q_ss * 2), lane);
+  if constexpr (CACHE) {
+    // Row r of the wave is query row_query(wrow0 + r), head row_head: offsets
+    // from the wave's first query (the host routes only strides whose offsets
+    // stay far below 2^31); rows past the last one lie beyond the resource.
+    const int i0 = row_query(wrow0);
+    const u32x4 rs = make_rsrc_words(qg + q_base + (int64_t)i0 * p.q_ss, 0x80000000u);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int r = 4 * i + (lane >> 4);
+      const int gr = wrow0 + r;
+      const uint32_t ro = (uint32_t)((row_query(gr) - i0) * (int)p.q_ss + row_head(gr) * (int)p.q_sh) * 2;
+      buf_load16_lds(rs, lds_address(q_st) + i * 1024,
+                     gr < rows ? ro + (uint32_t)(((lane & 15) ^ (r & 15)) * 16) : 0xfffffff0u);
+    }
+  } else {
+    stage_rows_load(make_rsrc_words(qg + q_base + (int64_t)wrow0 * p.q_ss,
+                                    rows_extent(wrow0, Sq, p.q_ss, D)),
+                    lds_address(q_st), (uint32_t)(p.q_ss * 2), lane);
+  }
   auto prescale_q = [&]() {
     if constexpr (kPre) {
       const float qs = p.scale_log2;
@@ -215,8 +352,9 @@ void prefill_pp_kernel(const FwdParams p) {
   for (int i = 0; i < IPW; ++i) {
     const int r = RPI * (IPW * w + i) + (lane >> 4);
     const int pc = lane & 15;
-    k_off[i] = (uint32_t)r * k_row_b + (uint32_t)((pc ^ (r & 15)) * 16);
-    v_off[i] = (uint32_t)r * v_row_b + (uint32_t)((pc ^ (4 * (r & 3))) * 16);
+    const int rr = PAGED ? r - RPI * IPW * w : r;   // paged: from the wave's first row
+    k_off[i] = (uint32_t)rr * k_row_b + (uint32_t)((pc ^ (r & 15)) * 16);
+    v_off[i] = (uint32_t)rr * v_row_b + (uint32_t)((pc ^ (4 * (r & 3))) * 16);
   }
   uint8_t* const k_lds = smem_pp;
   uint8_t* const v_lds = smem_pp + NS * TILEB;
@@ -225,10 +363,29 @@ void prefill_pp_kernel(const FwdParams p) {
   // (keeping the wait counts uniform) and writes zeros.
   const uint32_t k_lds_a = lds_address(k_lds) + IPW * w * 1024;
   const uint32_t v_lds_a = lds_address(v_lds) + IPW * w * 1024;
+  // Paged: first key of this wave's rows of tile rel, its page (-1 past the
+  // last key) and the resource that ends at the last valid one of its 8 rows.
+  auto wave_key = [&](int rel) __attribute__((always_inline)) {
+    return (t_begin + rel) * BN + RPI * IPW * w;
+  };
+  auto page_of = [&](int rel) __attribute__((always_inline)) {
+    const int n = wave_key(rel);
+    return rel < J && n < Sk ? bt_row[fdiv((uint32_t)n, p.fd_page)] : -1;
+  };
+  auto page_rsrc = [&](const uint16_t* base, int64_t sb, int64_t ss, int rel, int page)
+      __attribute__((always_inline)) {
+    const int n = wave_key(rel);
+    const bool live = page >= 0 && page < p.cache_blocks;   // page -1: no key of this tile is left
+    const int slot = live ? (int)fmod((uint32_t)n, p.fd_page) : 0;
+    return make_rsrc_words(base + (live ? (int64_t)page * sb + (int64_t)slot * ss : 0),
+                           live ? rows_extent(0, min(RPI * IPW, Sk - n), ss, D) : 0u);
+  };
+  int page_k = -1, page_v = -1;   // pages of the next K and V tile to load
   auto load_k = [&](int rel) {
     const int n0 = (t_begin + rel) * BN;
     const uint32_t ext = rel < J ? rows_extent(n0, Sk, p.k_ss, D) : 0u;
-    const u32x4 rs = make_rsrc_words(kg + (int64_t)(rel < J ? n0 : 0) * p.k_ss, ext);
+    const u32x4 rs = PAGED ? page_rsrc(kg, p.k_sb, p.k_ss, rel, page_k)
+                           : make_rsrc_words(kg + (int64_t)(rel < J ? n0 : 0) * p.k_ss, ext);
     const uint32_t dst = k_lds_a + (rel % NS) * TILEB;
 #pragma unroll
     for (int i = 0; i < IPW; ++i) buf_load16_lds(rs, dst + i * 1024, k_off[i]);
@@ -236,7 +393,8 @@ void prefill_pp_kernel(const FwdParams p) {
   auto load_v = [&](int rel) {
     const int n0 = (t_begin + rel) * BN;
     const uint32_t ext = rel < J ? rows_extent(n0, Sk, p.v_ss, D) : 0u;
-    const u32x4 rs = make_rsrc_words(vg + (int64_t)(rel < J ? n0 : 0) * p.v_ss, ext);
+    const u32x4 rs = PAGED ? page_rsrc(vg, p.v_sb, p.v_ss, rel, page_v)
+                           : make_rsrc_words(vg + (int64_t)(rel < J ? n0 : 0) * p.v_ss, ext);
     const uint32_t dst = v_lds_a + (rel % NS) * TILEB;
 #pragma unroll
     for (int i = 0; i < IPW; ++i) buf_load16_lds(rs, dst + i * 1024, v_off[i]);
@@ -391,7 +549,7 @@ void prefill_pp_kernel(const FwdParams p) {
     }
     const float mq4 = halves_max(fmaxf(fmaxf(mq[0], mq[1]), fmaxf(mq[2], mq[3])));
     const float mx = kPre ? mq4 + m_c : mq4 * sl;
-    const bool raise = mx > m_run + kRescaleSlack;
+    const bool raise = mx > m_run + kSlack;
     if (__builtin_amdgcn_ballot_w64(raise)) {
       const float m_new = raise ? mx : m_run;
       const float alpha = m_new == m_run ? 1.f : __builtin_amdgcn_exp2f(m_run - m_new);
@@ -421,7 +579,7 @@ void prefill_pp_kernel(const FwdParams p) {
         const float e0 = __builtin_amdgcn_exp2f(expo(sv[o8 + 2 * j]));
         const float e1 = __builtin_amdgcn_exp2f(expo(sv[o8 + 2 * j + 1]));
         pbuf[cc][j] = T::pack2(e0, e1);
-        if (T::kSumRounded)
+        if (kSumRounded)
           lq[j] = T::sum2(pbuf[cc][j], lq[j]);
         else
           lq[j] += e0 + e1;
@@ -432,10 +590,20 @@ void prefill_pp_kernel(const FwdParams p) {
 
   // ------------------------------------------------------------ prologue
   // Stages 0..NS-2 of K and 0..NS-3 of V; the Q rows retire with them.
+  if constexpr (PAGED) {
 #pragma unroll
-  for (int r = 0; r < NS - 1; ++r) load_k(r);
+    for (int r = 0; r < NS - 1; ++r) {
+      page_k = page_v = page_of(r);
+      load_k(r);
+      if (r < NS - 2) load_v(r);
+    }
+    page_k = page_of(NS - 1);   // (page_v: that of tile NS - 2)
+  } else {
 #pragma unroll
-  for (int r = 0; r < NS - 2; ++r) load_v(r);
+    for (int r = 0; r < NS - 1; ++r) load_k(r);
+#pragma unroll
+    for (int r = 0; r < NS - 2; ++r) load_v(r);
+  }
   __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
   pp_barrier();
   stage_rows_read_operand<NKC>(q_st, c32, g, qreg);
@@ -452,7 +620,14 @@ void prefill_pp_kernel(const FwdParams p) {
   auto softmax_step = [&](int j) {
     load_k(j + NS - 1);
     load_v(j + NS - 2);
+    if constexpr (PAGED) {
+      page_v = page_k;
+      page_k = page_of(j + NS);
+    }
     softmax_tile((t_begin + j) * BN, wave_masks(j));
+    // The table entry has arrived before the GEMM phase: a scalar load in
+    // flight there would turn every counted wait for LDS reads into a full one.
+    if constexpr (PAGED) asm volatile("" : "+s"(page_k));
     // This wave's loads from the previous softmax step have landed.
     __builtin_amdgcn_s_waitcnt(0x0f70 | (2 * IPW));
   };
@@ -481,10 +656,107 @@ void prefill_pp_kernel(const FwdParams p) {
   const float l_tot = halves_sum(l_run);
   const float inv_l = l_tot > 0.f ? 1.f / l_tot : 0.f;
   const float lse_val = l_tot > 0.f ? (m_run + __log2f(l_tot)) * kLn2 : -INFINITY;
-  stage_rows_store<T, NDB>(acc, inv_l, smem_pp + w * kStageOutBytes, c32, g, lane,
-                           static_cast<uint16_t*>(p.o) + o_base + (int64_t)wrow0 * p.o_ss,
-                           p.o_ss, Sq - wrow0);
-  if (p.lse != nullptr && g == 0 && row_valid) p.lse[lse_base + (int64_t)qi * p.lse_ss] = lse_val;
+  if constexpr (CACHE) {
+    uint16_t* const og = static_cast<uint16_t*>(p.o) + o_base;
+    if (Sk > p.split_tiles * BN) {
+      // One of several splits: the normalized fp32 rows, staged through LDS so
+      // that every store covers two whole 512-byte rows of the workspace.
+      static_assert(Tile::NW * kStagePartBytes <= Tile::LDS_BYTES, "partial rows must fit the LDS");
+      const int64_t prow0 = ((int64_t)split * p.batch + b) * Sq;
+      uint8_t* const st = smem_pp + w * kStagePartBytes;
+      stage_part_write<NDB>(acc, inv_l, st, c32, g);
+      const uint8_t* const rd = st + (lane >> 5) * kStagePartPitch + (lane & 31) * 16;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const f32x4 val = *reinterpret_cast<const f32x4*>(rd + i * 2 * kStagePartPitch);
+        const int gr = wrow0 + 2 * i + (lane >> 5);
+        if (gr < rows) {
+          const int64_t prow = (prow0 + row_query(gr)) * p.heads_q + hh + row_head(gr);
+          *reinterpret_cast<f32x4*>(p.o_part + prow * D + (lane & 31) * 4) = val;
+        }
+      }
+      if (g == 0 && row_valid)
+        p.lse_part[(prow0 + row_query(qi)) * p.heads_q + hh + row_head(qi)] = lse_val;
+      return;
+    }
+    u32x4 out[8];
+    stage_rows_gather<T, NDB>(acc, inv_l, smem_pp + w * kStageOutBytes, c32, g, lane, out);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int gr = wrow0 + 4 * i + (lane >> 4);
+      if (gr < rows)
+        store16(og + (int64_t)row_query(gr) * p.o_ss + (int64_t)row_head(gr) * p.o_sh + (lane & 15) * 8,
+                out[i]);
+    }
+    if (p.lse != nullptr && g == 0 && row_valid)
+      p.lse[lse_base + (int64_t)row_query(qi) * p.lse_ss + (int64_t)row_head(qi) * p.lse_sh] = lse_val;
+  } else {
+    stage_rows_store<T, NDB>(acc, inv_l, smem_pp + w * kStageOutBytes, c32, g, lane,
+                             static_cast<uint16_t*>(p.o) + o_base + (int64_t)wrow0 * p.o_ss,
+                             p.o_ss, Sq - wrow0);
+    if (p.lse != nullptr && g == 0 && row_valid) p.lse[lse_base + (int64_t)qi * p.lse_ss] = lse_val;
+  }
+}
+
+// Merge of the key splits of a KV-cache launch: out = sum_s exp(lse_s - lse)
+// o_s, lse = log sum_s exp(lse_s) over the splits that hold keys of the row's
+// sequence.  Sequences of one split were written by the split kernel.  One
+// thread per row and 4 dims, kCacheMergeBatch splits' loads in flight: bound
+// by reading the partials.
+constexpr int kCacheMergeBatch = 4;
+template <class T>
+__global__ __launch_bounds__(256) void cache_combine_kernel(const FwdParams p, int D) {
+  const int quads = D / 4;
+  const int64_t nrows = (int64_t)p.batch * p.seqlen_q * p.heads_q;
+  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (idx >= nrows * quads) return;
+  const int64_t row = idx / quads;
+  const int qd = (int)(idx % quads);
+  const int h = (int)(row % p.heads_q);
+  const int i = (int)((row / p.heads_q) % p.seqlen_q);
+  const int b = (int)(row / ((int64_t)p.heads_q * p.seqlen_q));
+  int crow, pad;
+  const int L = cache_keys(p, b, &crow, &pad);
+  const int split_keys = p.split_tiles * 64;
+  if (L <= split_keys) return;
+  const int n = min(p.num_splits, (L + split_keys - 1) / split_keys);
+  float m = -INFINITY, tot = 0.f;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < n; s0 += kCacheMergeBatch) {
+    float ls[kCacheMergeBatch];
+    f32x4 o[kCacheMergeBatch];
+#pragma unroll
+    for (int u = 0; u < kCacheMergeBatch; ++u) {
+      const int s = s0 + u;
+      ls[u] = s < n ? p.lse_part[(int64_t)s * nrows + row] : -INFINITY;
+      o[u] = s < n ? *reinterpret_cast<const f32x4*>(p.o_part + ((int64_t)s * nrows + row) * D + qd * 4)
+                   : f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    float mb = m;
+#pragma unroll
+    for (int u = 0; u < kCacheMergeBatch; ++u) mb = fmaxf(mb, ls[u]);
+    if (mb == -INFINITY) continue;
+    const float rescale = __expf(m - mb);   // m == -inf -> 0
+    tot *= rescale;
+    acc *= rescale;
+#pragma unroll
+    for (int u = 0; u < kCacheMergeBatch; ++u) {
+      const float wgt = ls[u] == -INFINITY ? 0.f : __expf(ls[u] - mb);
+      tot += wgt;
+      acc += wgt * o[u];
+    }
+    m = mb;
+  }
+  const float inv = tot > 0.f ? 1.f / tot : 0.f;
+  uint16_t* orow = static_cast<uint16_t*>(p.o) + (int64_t)b * p.o_sb + (int64_t)i * p.o_ss +
+                   (int64_t)h * p.o_sh;
+  u32x2 val;
+  val[0] = T::pack2(acc[0] * inv, acc[1] * inv);
+  val[1] = T::pack2(acc[2] * inv, acc[3] * inv);
+  *reinterpret_cast<u32x2*>(orow + qd * 4) = val;
+  if (p.lse != nullptr && qd == 0)
+    p.lse[(int64_t)b * p.lse_sb + (int64_t)i * p.lse_ss + (int64_t)h * p.lse_sh] =
+        tot > 0.f ? m + __logf(tot) : -INFINITY;
 }
 
 }  // namespace fa

@@ -79,6 +79,27 @@ __device__ inline void stage_rows_put(const u32x4* rows, uint16_t* orow0, int64_
   }
 }
 
+// The same accumulators times inv_l as fp32 rows of 32 NDB values, written to a
+// staging area of kStagePartBytes with rows kStagePartPitch bytes apart (head
+// dim 128); the caller reads whole rows back.
+constexpr int kStagePartPitch = 528;
+constexpr int kStagePartBytes = 32 * kStagePartPitch;
+template <int NDB>
+__device__ inline void stage_part_write(const f32x16* acc, float inv_l, uint8_t* st, int c32, int g) {
+  uint8_t* const wr = st + c32 * kStagePartPitch + 16 * g;
+#pragma unroll
+  for (int db = 0; db < NDB; ++db) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      *reinterpret_cast<f32x4*>(wr + (db * 32 + 8 * r) * 4) =
+          f32x4{acc[db][4 * r] * inv_l, acc[db][4 * r + 1] * inv_l, acc[db][4 * r + 2] * inv_l,
+                acc[db][4 * r + 3] * inv_l};
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 template <class T, int NDB>
 __device__ inline void stage_rows_store(const f32x16* acc, float inv_l, uint8_t* st, int c32,
                                         int g, int lane, uint16_t* orow0, int64_t o_ss,
