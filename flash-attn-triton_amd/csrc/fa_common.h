@@ -152,13 +152,13 @@ __device__ inline void work_item(int L, int total, int n_mblocks, bool heavy_fir
   if (heavy_first && total % (kXcds * n_mblocks) == 0) {
     const int groups_per_xcd = total / kXcds / n_mblocks;
     const int w = span <= 0 || span > groups_per_xcd ? groups_per_xcd : span;
-    if (groups_per_xcd % w == 0) {
-      const int k = L / kXcds;
-      const int r = k % (w * n_mblocks);
-      mb = n_mblocks - 1 - r / w;
-      grp = (L % kXcds) * groups_per_xcd + (k / (w * n_mblocks)) * w + r % w;
-      return;
-    }
+    const int k = L / kXcds;
+    const int g0 = k / (w * n_mblocks) * w;        // first group of this span
+    const int gw = min(w, groups_per_xcd - g0);    // (the last span may be narrower)
+    const int r = k - g0 * n_mblocks;
+    mb = n_mblocks - 1 - r / gw;
+    grp = (L % kXcds) * groups_per_xcd + g0 + r % gw;
+    return;
   }
   const int id = xcd_remap(L, total);
   mb = id % n_mblocks;

@@ -76,7 +76,7 @@ struct FwdParams {
   int kv_causal_offset;
   int num_splits, split_tiles;
   float* o_part; float* lse_part;
-  int n_mblocks, total_blocks, heavy_first;
+  int n_mblocks, total_blocks, heavy_first, span;   // span: work_item's (prefill_d64_kernel)
   // prefill_persist_kernel: row blocks per workgroup, and divisions by the
   // row blocks (causal: pairs of row blocks) per group, the query heads and
   // the GQA group size (set by the persistent launchers).

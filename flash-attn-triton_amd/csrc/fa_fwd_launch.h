@@ -6,6 +6,7 @@
 #include "fa_prefill_kernel.h"
 #include "fa_prefill_pp.h"
 #include "fa_prefill_persist.h"
+#include "fa_prefill_d64.h"
 
 namespace fa {
 
@@ -40,7 +41,8 @@ hipError_t launch_fwd_cfg(FwdParams p, int rows_for_grid, int outer_blocks, hipS
 //                      by LDS-DMA through a 3 K / 2 V stage ring (KS = 3)
 //   D = 128, unmasked: 8 waves (256 query rows share each K/V tile), 64-key tiles
 //   D = 256          : 8 waves, 32-key tiles (the O^T accumulators take 128 VGPRs)
-//   D = 32 / 64      : 4 waves, 64-key tiles
+//   D = 32 / 64      : 4 waves, 64-key tiles (64 with the generic epilogue or
+//                      attn_bias only: fa_prefill_d64.h has the plain one)
 // Measured on MI355X at B4 H32 S4096 D128: the masked choice is ahead on
 // causal and varlen (less work past the diagonal / sequence end), the
 // unmasked one on non-causal.
@@ -127,13 +129,16 @@ hipError_t launch_prefill_persist(FwdParams p, hipStream_t st, bool* launched) {
   return hipGetLastError();
 }
 
-// Paged keys the ping-pong kernel's 8-row tile loads can take.
-inline bool pp_pages(const FwdParams& p) { return p.block_table != nullptr && p.page_size % 8 == 0; }
+// Paged keys whose pages hold whole groups of the rows one wave copies: 8 on
+// the ping-pong kernel (head dim 128), 16 on prefill_d64_kernel.
+inline bool pp_pages(const FwdParams& p, int head_dim) {
+  return p.block_table != nullptr && p.page_size % (head_dim == 64 ? 16 : 8) == 0;
+}
 
-// KV-cache launches that run on the ping-pong kernel instead of fwd_kernel:
-// head dim 128, more rows than the decode kernel's 32, pages of whole 8-row
-// groups, strides whose 32-row offsets stay far inside 32 bits, and neither
-// ALiBi nor a scale <= 0 (`generic`).  Ahead over the whole of that range:
+// KV-cache launches that run on the ping-pong kernel (head dim 128) or
+// prefill_d64_kernel (64) instead of fwd_kernel: more rows than the decode
+// kernel's 32, pages as above, strides whose 32-row offsets stay far inside 32
+// bits, and neither ALiBi nor a scale <= 0 (`generic`).  Ahead over the whole of that range:
 // per call with fwd_kernel and with it, bf16, MI355X, 512 queries and 32 / 8
 // heads 614 -> 168 us; 33 rows per KV head (the fewest; 32 KV heads, B8) 515 ->
 // 192 us; 64 queries (B4) 135 -> 102 us, where the host's argument checks bound
@@ -141,9 +146,40 @@ inline bool pp_pages(const FwdParams& p) { return p.block_table != nullptr && p.
 inline bool cache_pp_route(const FwdParams& p, int head_dim, bool generic) {
   constexpr int64_t kMaxStride = (int64_t)1 << 24;   // elements
   const int64_t rows = (int64_t)p.seqlen_q * p.group;
-  return head_dim == 128 && !generic && rows > 32 && (p.block_table == nullptr || pp_pages(p)) &&
+  return (head_dim == 128 || head_dim == 64) && !generic && rows > 32 &&
+         (p.block_table == nullptr || pp_pages(p, head_dim)) &&
          p.q_ss <= kMaxStride && p.q_sh * p.group <= kMaxStride && p.k_ss <= kMaxStride &&
          p.v_ss <= kMaxStride;
+}
+
+// Head dim 64, plain epilogue (fa_prefill_d64.h): 4 waves, 128 rows per
+// workgroup.  Causal launches interleave `span` groups per XCD heaviest block
+// first: a narrow span leaves the last group's heavy blocks to the end of the
+// launch, a wide one streams more K/V than the 4 MiB L2 holds.  8 groups at
+// S = 4096 (8 MiB), all 16 at 1024 (4 MiB) were best; measured on one MI355X
+// for spans 1 / 4 / 8 / 16, fp16, B / S / Hq / Hk: 8 / 1024 / 16 / 16 39.0 /
+// 37.4 / 35.6 / 33.9 us, 4 / 2048 / 32 / 32 108 / 96 / 93 / 93, 2 / 3001 / 32 /
+// 8 (8 groups) 115 / 104 / 93, 4 / 4096 / 32 / 32 353 / 324 / 316 / 324.
+template <class T, int MODE, bool PAGED>
+hipError_t launch_prefill_d64(FwdParams p, hipStream_t st) {
+  using Tile = D64Tile;
+  auto kern = prefill_d64_kernel<T, MODE, PAGED>;
+  static std::atomic<uint64_t> lds_devices{0};
+  if (hipError_t e = set_lds_limit(lds_devices, kern, Tile::LDS_BYTES); e != hipSuccess) return e;
+  const int rows = MODE == kPpCache ? p.seqlen_q * p.group : p.seqlen_q;
+  p.n_mblocks = (rows + Tile::BM - 1) / Tile::BM;
+  int64_t total = (int64_t)p.n_mblocks * p.heads_q * p.batch;
+  if (MODE == kPpCache) {
+    total = (int64_t)p.n_mblocks * p.heads_k * p.batch * p.num_splits;
+    p.fd_group = make_fastdiv((uint32_t)p.group);
+  }
+  if (PAGED) p.fd_page = make_fastdiv((uint32_t)p.page_size);
+  if (total <= 0) return hipSuccess;
+  if (total > 0x7fffffff) return hipErrorInvalidConfiguration;
+  p.total_blocks = (int)total;
+  p.span = p.seqlen_k > 0 && p.seqlen_k < 4096 ? 32768 / p.seqlen_k : 8;
+  hipLaunchKernelGGL(kern, dim3((unsigned)total), dim3(Tile::NT), Tile::LDS_BYTES, st, p);
+  return hipGetLastError();
 }
 
 template <class T, int D, bool GEN>
@@ -187,6 +223,13 @@ hipError_t launch_prefill(const FwdParams& p, hipStream_t st) {
     return launch_prefill_cfg<T, D, 8, 64, GEN, 2>(p, st);
   } else if constexpr (D == 256) {
     return launch_prefill_cfg<T, D, 8, 32, GEN, 2>(p, st);
+  } else if constexpr (D == 64) {
+    if constexpr (!GEN) {
+      if (p.cu_q != nullptr) return launch_prefill_d64<T, kPpVarlen, false>(p, st);
+      return launch_prefill_d64<T, kPpDense, false>(p, st);
+    } else {
+      return launch_prefill_cfg<T, D, 4, 64, GEN, 2>(p, st);
+    }
   } else {
     return launch_prefill_cfg<T, D, 4, 64, GEN, 2>(p, st);
   }
@@ -199,7 +242,10 @@ hipError_t launch_fwd_d(const FwdParams& p, hipStream_t st) {
     // per key on the general one.
     if (p.block_table != nullptr) {
       if constexpr (D == 128 && !GEN) {
-        if (pp_pages(p)) return launch_prefill_pp<T, D, kPpVarlen, true>(p, st);
+        if (pp_pages(p, D)) return launch_prefill_pp<T, D, kPpVarlen, true>(p, st);
+      }
+      if constexpr (D == 64 && !GEN) {
+        if (pp_pages(p, D)) return launch_prefill_d64<T, kPpVarlen, true>(p, st);
       }
       using C = PrefillCfg<D>;
       return launch_fwd_cfg<T, D, C::NW, C::BN, MODE, GEN>(p, p.seqlen_q, p.heads_q * p.batch, st);
@@ -215,6 +261,11 @@ hipError_t launch_fwd_d(const FwdParams& p, hipStream_t st) {
     if (p.cache_pp)
       return p.block_table != nullptr ? launch_prefill_pp<T, D, kPpCache, true>(p, st)
                                       : launch_prefill_pp<T, D, kPpCache, false>(p, st);
+  }
+  if constexpr (D == 64 && !GEN) {
+    if (p.cache_pp)
+      return p.block_table != nullptr ? launch_prefill_d64<T, kPpCache, true>(p, st)
+                                      : launch_prefill_d64<T, kPpCache, false>(p, st);
   }
   const int rows = p.seqlen_q * p.group;
   const int outer = p.heads_k * p.batch * p.num_splits;

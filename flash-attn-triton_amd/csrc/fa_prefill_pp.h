@@ -661,14 +661,14 @@ void prefill_pp_kernel(const FwdParams p) {
     if (Sk > p.split_tiles * BN) {
       // One of several splits: the normalized fp32 rows, staged through LDS so
       // that every store covers two whole 512-byte rows of the workspace.
-      static_assert(Tile::NW * kStagePartBytes <= Tile::LDS_BYTES, "partial rows must fit the LDS");
+      static_assert(Tile::NW * stage_part_bytes(NDB) <= Tile::LDS_BYTES, "partial rows must fit the LDS");
       const int64_t prow0 = ((int64_t)split * p.batch + b) * Sq;
-      uint8_t* const st = smem_pp + w * kStagePartBytes;
+      uint8_t* const st = smem_pp + w * stage_part_bytes(NDB);
       stage_part_write<NDB>(acc, inv_l, st, c32, g);
-      const uint8_t* const rd = st + (lane >> 5) * kStagePartPitch + (lane & 31) * 16;
+      const uint8_t* const rd = st + (lane >> 5) * stage_part_pitch(NDB) + (lane & 31) * 16;
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
-        const f32x4 val = *reinterpret_cast<const f32x4*>(rd + i * 2 * kStagePartPitch);
+        const f32x4 val = *reinterpret_cast<const f32x4*>(rd + i * 2 * stage_part_pitch(NDB));
         const int gr = wrow0 + 2 * i + (lane >> 5);
         if (gr < rows) {
           const int64_t prow = (prow0 + row_query(gr)) * p.heads_q + hh + row_head(gr);

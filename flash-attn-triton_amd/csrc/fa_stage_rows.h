@@ -37,17 +37,19 @@ __device__ inline void stage_rows_read_operand(const uint8_t* st, int c32, int g
 
 // O^T accumulators (lane (c32, g): dims 32 db + 8 (v / 4) + 4 g + v % 4 of row
 // c32) times inv_l, packed to 16 bits, written to a staging area of
-// kStageOutBytes and read back as whole rows: out[i] is chunk lane % 16 of row
-// 4 i + lane / 16.  Rows are kStageOutPitch bytes apart (one 16-byte pad per
-// 256-byte row spreads the 32 rows of a write over the banks), so every LDS
-// address is a per-lane base plus an immediate (a swizzle would need one
-// register per chunk).
-constexpr int kStageOutPitch = 272;
-constexpr int kStageOutBytes = 32 * kStageOutPitch;
+// stage_out_bytes and read back as whole rows of 4 NDB 16-byte chunks: out[i]
+// is the chunk lane % (4 NDB) of row i * 16 / NDB + lane / (4 NDB).  Rows are
+// one 16-byte pad apart (it spreads the 32 rows of a write over the banks), so
+// every LDS address is a per-lane base plus an immediate (a swizzle would need
+// one register per chunk).
+constexpr int stage_out_pitch(int ndb) { return ndb * 64 + 16; }
+constexpr int stage_out_bytes(int ndb) { return 32 * stage_out_pitch(ndb); }
+constexpr int kStageOutBytes = stage_out_bytes(4);   // head dim 128
 template <class T, int NDB>
 __device__ inline void stage_rows_gather(const f32x16* acc, float inv_l, uint8_t* st, int c32,
                                          int g, int lane, u32x4* out) {
-  uint8_t* const wr = st + c32 * kStageOutPitch + 8 * g;
+  constexpr int kPitch = stage_out_pitch(NDB), kCpr = 4 * NDB, kRows = 64 / kCpr;
+  uint8_t* const wr = st + c32 * kPitch + 8 * g;
 #pragma unroll
   for (int db = 0; db < NDB; ++db) {
 #pragma unroll
@@ -62,31 +64,33 @@ __device__ inline void stage_rows_gather(const f32x16* acc, float inv_l, uint8_t
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  const uint8_t* const rd = st + (lane >> 4) * kStageOutPitch + (lane & 15) * 16;
+  const uint8_t* const rd = st + (lane / kCpr) * kPitch + (lane % kCpr) * 16;
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
-    out[i] = *reinterpret_cast<const u32x4*>(rd + i * 4 * kStageOutPitch);
+  for (int i = 0; i < 32 / kRows; ++i)
+    out[i] = *reinterpret_cast<const u32x4*>(rd + i * kRows * kPitch);
 }
 
 // Stores of stage_rows_gather's rows [0, rows_ok) at `orow0` (row stride
-// o_ss elements): four whole rows per instruction.
+// o_ss elements): whole rows, 1 KiB per instruction.
+template <int NDB = 4>
 __device__ inline void stage_rows_put(const u32x4* rows, uint16_t* orow0, int64_t o_ss, int lane,
                                       int rows_ok = 32) {
+  constexpr int kCpr = 4 * NDB, kRows = 64 / kCpr;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int r = 4 * i + (lane >> 4);
-    if (r < rows_ok) store16(orow0 + (int64_t)r * o_ss + (lane & 15) * 8, rows[i]);
+  for (int i = 0; i < 32 / kRows; ++i) {
+    const int r = kRows * i + lane / kCpr;
+    if (r < rows_ok) store16(orow0 + (int64_t)r * o_ss + (lane % kCpr) * 8, rows[i]);
   }
 }
 
 // The same accumulators times inv_l as fp32 rows of 32 NDB values, written to a
-// staging area of kStagePartBytes with rows kStagePartPitch bytes apart (head
-// dim 128); the caller reads whole rows back.
-constexpr int kStagePartPitch = 528;
-constexpr int kStagePartBytes = 32 * kStagePartPitch;
+// staging area of stage_part_bytes with rows stage_part_pitch bytes apart; the
+// caller reads whole rows back.
+constexpr int stage_part_pitch(int ndb) { return ndb * 128 + 16; }
+constexpr int stage_part_bytes(int ndb) { return 32 * stage_part_pitch(ndb); }
 template <int NDB>
 __device__ inline void stage_part_write(const f32x16* acc, float inv_l, uint8_t* st, int c32, int g) {
-  uint8_t* const wr = st + c32 * kStagePartPitch + 16 * g;
+  uint8_t* const wr = st + c32 * stage_part_pitch(NDB) + 16 * g;
 #pragma unroll
   for (int db = 0; db < NDB; ++db) {
 #pragma unroll
@@ -104,9 +108,9 @@ template <class T, int NDB>
 __device__ inline void stage_rows_store(const f32x16* acc, float inv_l, uint8_t* st, int c32,
                                         int g, int lane, uint16_t* orow0, int64_t o_ss,
                                         int rows_ok) {
-  u32x4 rows[8];
+  u32x4 rows[2 * NDB];
   stage_rows_gather<T, NDB>(acc, inv_l, st, c32, g, lane, rows);
-  stage_rows_put(rows, orow0, o_ss, lane, rows_ok);
+  stage_rows_put<NDB>(rows, orow0, o_ss, lane, rows_ok);
 }
 
 }  // namespace fa
