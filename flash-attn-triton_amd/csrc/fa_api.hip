@@ -295,7 +295,7 @@ int fa_fwd_dense(const void* q, const void* k, const void* v, void* out, float* 
                     "fa_fwd_dense launch");
 }
 
-int fa_fwd_varlen(const void* q, const void* k, const void* v, void* out, float* lse,
+int fa_fwd_varlen_guarded(const void* q, const void* k, const void* v, void* out, float* lse,
                   const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, int64_t batch,
                   int64_t max_seqlen_q, int64_t max_seqlen_k, int64_t heads_q, int64_t heads_k,
                   int64_t head_dim, const int64_t* q_stride, const int64_t* k_stride,
@@ -306,7 +306,10 @@ int fa_fwd_varlen(const void* q, const void* k, const void* v, void* out, float*
                   const int32_t* seqused_k, const int32_t* cu_seqlens_out,
                   const int32_t* block_table, int64_t block_table_stride, int64_t page_size,
                   int64_t num_pages, int64_t block_table_cols, float dropout_p,
-                  uint64_t dropout_seed, fa_stream_t stream) {
+                  uint64_t dropout_seed, const int32_t* guard, int guard_n,
+                  fa_stream_t stream) {
+  if (guard_n < 0 || (guard_n > 0 && !guard))
+    return fail(FA_ERR_INVALID, "fa_fwd_varlen_guarded: guard_n without guard");
   if (!q || !k || !v || !out || !cu_seqlens_q || !cu_seqlens_k || !q_stride || !k_stride ||
       !v_stride || !o_stride)
     return fail(FA_ERR_INVALID, "fa_fwd_varlen: null pointer argument");
@@ -348,6 +351,7 @@ int fa_fwd_varlen(const void* q, const void* k, const void* v, void* out, float*
   if (lse) { p.lse_ss = lse_stride[0]; p.lse_sh = lse_stride[1]; }
   p.cu_q = cu_seqlens_q; p.cu_k = cu_seqlens_k;
   p.seqused_q = seqused_q; p.seqused_k = seqused_k; p.cu_o = cu_seqlens_out;
+  p.guard = guard; p.guard_n = guard_n;
   if (!fill_dropout(p.drop, dropout_p, dropout_seed))
     return fail(FA_ERR_INVALID, "fa_fwd_varlen: dropout_p must be in [0, 1 - 2^-17]");
   p.batch = (int)batch; p.seqlen_q = (int)max_seqlen_q; p.seqlen_k = (int)max_seqlen_k;
@@ -362,6 +366,27 @@ int fa_fwd_varlen(const void* q, const void* k, const void* v, void* out, float*
   return hip_status(launch_fwd(dtype, p, fa::kModePrefill, (int)head_dim, needs_generic(p),
                                (hipStream_t)stream),
                     "fa_fwd_varlen launch");
+}
+
+int fa_fwd_varlen(const void* q, const void* k, const void* v, void* out, float* lse,
+                  const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, int64_t batch,
+                  int64_t max_seqlen_q, int64_t max_seqlen_k, int64_t heads_q, int64_t heads_k,
+                  int64_t head_dim, const int64_t* q_stride, const int64_t* k_stride,
+                  const int64_t* v_stride, const int64_t* o_stride, const int64_t* lse_stride,
+                  int dtype, float softmax_scale, int causal, int64_t window_left,
+                  int64_t window_right, float softcap, const float* alibi_slopes,
+                  int64_t alibi_batch_stride, const int32_t* seqused_q,
+                  const int32_t* seqused_k, const int32_t* cu_seqlens_out,
+                  const int32_t* block_table, int64_t block_table_stride, int64_t page_size,
+                  int64_t num_pages, int64_t block_table_cols, float dropout_p,
+                  uint64_t dropout_seed, fa_stream_t stream) {
+  return fa_fwd_varlen_guarded(q, k, v, out, lse, cu_seqlens_q, cu_seqlens_k, batch, max_seqlen_q,
+                               max_seqlen_k, heads_q, heads_k, head_dim, q_stride, k_stride,
+                               v_stride, o_stride, lse_stride, dtype, softmax_scale, causal,
+                               window_left, window_right, softcap, alibi_slopes,
+                               alibi_batch_stride, seqused_q, seqused_k, cu_seqlens_out,
+                               block_table, block_table_stride, page_size, num_pages,
+                               block_table_cols, dropout_p, dropout_seed, nullptr, 0, stream);
 }
 
 int fa_bwd_dense(const void* q, const void* k, const void* v, const void* out, const void* dout,
@@ -751,6 +776,72 @@ int fa_rotary_q(const void* q, void* out, const int32_t* cache_seqlens,
   p.interleaved = rotary_interleaved != 0; p.table_rows = rotary_rows;
   p.batch = (int)batch; p.seqlen_q = (int)seqlen_q; p.heads = (int)heads; p.head_dim = (int)head_dim;
   return hip_status(fa_launch_rotary_q(dtype, p, (hipStream_t)stream), "fa_rotary_q launch");
+}
+
+int fa_kvcache_update(const void* k_new, const void* v_new, void* k_cache, void* v_cache,
+                      const int32_t* cache_seqlens, const int32_t* block_table,
+                      int64_t block_table_stride, int64_t page_size, int64_t num_pages,
+                      const int32_t* cache_batch_idx, int64_t cache_rows,
+                      const int32_t* cache_leftpad, int64_t capacity, const void* rotary_cos,
+                      const void* rotary_sin, int table_dtype, int64_t rotary_dim,
+                      int64_t rotary_rows, int rotary_interleaved, const void* q, void* q_out,
+                      int64_t seqlen_q, int64_t heads_q, int32_t* lens_out, int64_t batch,
+                      int64_t n_new, int64_t heads_k, int64_t head_dim,
+                      const int64_t* k_new_stride, const int64_t* v_new_stride,
+                      const int64_t* k_cache_stride, const int64_t* v_cache_stride,
+                      const int64_t* q_stride, const int64_t* q_out_stride, int dtype,
+                      const int32_t* guard, int guard_n, fa_stream_t stream) {
+  const char* name = "fa_kvcache_update";
+  if (!cache_seqlens || (n_new > 0 && (!k_new || !v_new || !k_cache || !v_cache || !k_new_stride ||
+                                       !v_new_stride || !k_cache_stride || !v_cache_stride)))
+    return fail(FA_ERR_INVALID, "%s: null pointer argument", name);
+  if ((rotary_cos == nullptr) != (rotary_sin == nullptr) ||
+      (rotary_cos && (!q || !q_out || !q_stride || !q_out_stride)))
+    return fail(FA_ERR_INVALID, "%s: rotary_cos, rotary_sin, q and q_out go together", name);
+  if (!supported_dtype(dtype) || (rotary_cos && !supported_dtype(table_dtype)))
+    return fail(FA_ERR_UNSUPPORTED, "%s: dtype %d / table dtype %d not supported", name, dtype,
+                table_dtype);
+  if (batch < 0 || n_new < 0 || heads_k <= 0 || head_dim <= 0 || capacity < 0 || seqlen_q < 0 ||
+      (rotary_cos && heads_q <= 0) || guard_n < 0 || (guard_n > 0 && !guard) ||
+      (n_new > 0 && ((block_table && (page_size <= 0 || num_pages <= 0)) ||
+                     (!block_table && cache_rows <= 0))))
+    return fail(FA_ERR_INVALID, "%s: bad sizes", name);
+  if (rotary_cos && (rotary_dim <= 0 || rotary_dim % 2 != 0 || rotary_dim > head_dim ||
+                     rotary_rows <= 0))
+    return fail(FA_ERR_INVALID, "%s: rotary_dim %lld must be even, positive and at most head_dim",
+                name, (long long)rotary_dim);
+  if (batch * n_new * heads_k * head_dim > INT64_C(1) << 40 ||
+      batch * seqlen_q * heads_q * head_dim > INT64_C(1) << 40 || capacity > kMaxLen)
+    return fail(FA_ERR_UNSUPPORTED, "%s: sizes too large", name);
+  fa::UpdateParams u{};
+  fa::AppendParams& p = u.a;
+  p.seqlens = cache_seqlens; p.batch = (int)batch; p.n_new = (int)n_new;
+  p.heads_k = (int)heads_k; p.head_dim = (int)head_dim;
+  p.rot = (int)rotary_dim; p.interleaved = rotary_interleaved != 0; p.table_rows = rotary_rows;
+  if (n_new > 0) {
+    p.k_new = k_new; p.v_new = v_new; p.k_cache = k_cache; p.v_cache = v_cache;
+    p.kn_sb = k_new_stride[0]; p.kn_ss = k_new_stride[1]; p.kn_sh = k_new_stride[2];
+    p.vn_sb = v_new_stride[0]; p.vn_ss = v_new_stride[1]; p.vn_sh = v_new_stride[2];
+    p.kc_sb = k_cache_stride[0]; p.kc_ss = k_cache_stride[1]; p.kc_sh = k_cache_stride[2];
+    p.vc_sb = v_cache_stride[0]; p.vc_ss = v_cache_stride[1]; p.vc_sh = v_cache_stride[2];
+    p.block_table = block_table; p.bt_stride = block_table_stride;
+    p.page_size = (int)page_size; p.num_pages = (int)num_pages;
+    p.cache_rows = cache_batch_idx; p.cache_rows_n = (int)cache_rows; p.leftpad = cache_leftpad;
+    p.capacity = capacity;
+  }
+  if (rotary_cos) {
+    u.cos = rotary_cos; u.sin = rotary_sin; u.table_dtype = table_dtype;
+    fa::RotaryQParams& r = u.q;
+    r.q = q; r.out = q_out;
+    r.q_sb = q_stride[0]; r.q_ss = q_stride[1]; r.q_sh = q_stride[2];
+    r.o_sb = q_out_stride[0]; r.o_ss = q_out_stride[1]; r.o_sh = q_out_stride[2];
+    r.seqlens = cache_seqlens; r.leftpad = cache_leftpad;
+    r.rot = p.rot; r.interleaved = p.interleaved; r.table_rows = rotary_rows;
+    r.batch = (int)batch; r.seqlen_q = (int)seqlen_q; r.heads = (int)heads_q; r.head_dim = (int)head_dim;
+  }
+  u.lens_out = lens_out;
+  u.guard = guard; u.guard_n = guard_n;
+  return hip_status(fa_launch_kv_update(dtype, u, (hipStream_t)stream), "fa_kvcache_update launch");
 }
 
 int fa_quant_k_int8(const void* k, int8_t* k8, float* s_k, int64_t batch, int64_t heads,

@@ -85,6 +85,7 @@ void fwd_f32_kernel(const FwdParams p) {
   int kvh;
   if (MODE == kModePrefill) {
     kvh = hh / p.group;
+    if (guard_failed(p)) return;
     if (p.cu_q != nullptr) {
       const int qs = p.cu_q[b], ks = p.cu_k[b];
       Sq = p.cu_q[b + 1] - qs;

@@ -87,9 +87,20 @@ struct FwdParams {
   // (division by page_size).
   int cache_pp;
   FastDiv fd_page;
+  // Varlen launches issued before the host has read the checks of cu_seqlens:
+  // guard[0 .. guard_n) (device, written by fa_check_bounds) must all be zero.
+  const int* guard; int guard_n;
   // Dropout of the probabilities (prefill, GENERIC instantiations only).
   DropoutCfg drop;
 };
+
+// True when a check this launch is guarded by has failed: the kernel must
+// return without reading what was checked.
+__device__ inline bool guard_failed(const FwdParams& p) {
+  int bad = 0;
+  for (int i = 0; i < p.guard_n; ++i) bad |= p.guard[i];
+  return bad != 0;
+}
 
 template <int D, int NW, int BN>
 struct FwdTile {
@@ -152,6 +163,7 @@ void fwd_kernel(const FwdParams p) {
   const uint16_t* vg = static_cast<const uint16_t*>(p.v);
   uint16_t* og = static_cast<uint16_t*>(p.o);
 
+  if (MODE == kModePrefill && guard_failed(p)) return;
   int Sq, Sk;
   int64_t qoff = 0;
   int64_t q_base, o_base, lse_base;

@@ -25,7 +25,20 @@ struct RotaryQParams {
   int batch, seqlen_q, heads, head_dim;
 };
 
+// The append and the query rotation in one launch (either may be empty).  The
+// tables come in their own type (table_dtype: FA_DTYPE_*) and are rounded to
+// the element type as they are read; lens_out (nullable) receives
+// cache_seqlens + n_new; guard: see fa_check_bounds.
+struct UpdateParams {
+  AppendParams a;
+  RotaryQParams q;
+  const void* cos; const void* sin; int table_dtype;
+  int* lens_out;
+  const int* guard; int guard_n;
+};
+
 }  // namespace fa
 
+hipError_t fa_launch_kv_update(int dtype, const fa::UpdateParams& p, hipStream_t st);
 hipError_t fa_launch_kv_append(int dtype, const fa::AppendParams& p, hipStream_t st);
 hipError_t fa_launch_rotary_q(int dtype, const fa::RotaryQParams& p, hipStream_t st);

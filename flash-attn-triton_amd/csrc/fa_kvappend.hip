@@ -43,9 +43,23 @@ __device__ inline void st(void* base, int64_t i, float x) {
   else static_cast<uint16_t*>(base)[i] = (uint16_t)(T::pack2(x, 0.f) & 0xffffu);
 }
 
+// Rotary tables in their own type, read as the element type T holds them.
+template <class T>
+struct Table {
+  const void* base;
+  int dtype;
+  int64_t at;
+  __device__ inline float operator[](int j) const {
+    const float x = dtype == 2 ? ld<float>(base, at + j)
+                    : dtype == 1 ? ld<BF16>(base, at + j) : ld<F16>(base, at + j);
+    if constexpr (std::is_same<T, float>::value) return x;
+    else return T::to_float((uint16_t)(T::pack2(x, 0.f) & 0xffffu));
+  }
+};
+
 // Element d of the rotated row: `row(j)` reads element j of the source row.
-template <class F>
-__device__ inline float rotate(F row, int d, const float* cs, const float* sn, int rot, int inter) {
+template <class F, class C>
+__device__ inline float rotate(F row, int d, C cs, C sn, int rot, int inter) {
   if (d >= rot) return row(d);
   if (inter) {
     const int j = d >> 1;
@@ -57,9 +71,9 @@ __device__ inline float rotate(F row, int d, const float* cs, const float* sn, i
 
 }  // namespace
 
-template <class T>
-__global__ __launch_bounds__(256) void kv_append_kernel(const AppendParams p) {
-  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
+// Element idx of the append; `tables(pos)` gives row pos of {cos, sin}.
+template <class T, class F>
+__device__ inline void append_element(const AppendParams& p, int64_t idx, bool rotary, F tables) {
   const int64_t total = (int64_t)p.batch * p.n_new * p.heads_k * p.head_dim;
   if (idx >= total) return;
   const int d = (int)(idx % p.head_dim);
@@ -87,11 +101,10 @@ __global__ __launch_bounds__(256) void kv_append_kernel(const AppendParams p) {
   const int64_t kn = (int64_t)b * p.kn_sb + (int64_t)t * p.kn_ss + (int64_t)h * p.kn_sh;
   const int64_t vn = (int64_t)b * p.vn_sb + (int64_t)t * p.vn_ss + (int64_t)h * p.vn_sh + d;
   float kx;
-  if (p.cos != nullptr) {
+  if (rotary) {
     if (pos >= p.table_rows) return;
-    const int half = p.rot >> 1;
-    kx = rotate([&](int j) { return ld<T>(p.k_new, kn + j); }, d, p.cos + pos * half,
-                p.sin + pos * half, p.rot, p.interleaved);
+    const auto t2 = tables(pos * (p.rot >> 1));
+    kx = rotate([&](int j) { return ld<T>(p.k_new, kn + j); }, d, t2.c, t2.s, p.rot, p.interleaved);
   } else {
     kx = ld<T>(p.k_new, kn + d);
   }
@@ -99,9 +112,10 @@ __global__ __launch_bounds__(256) void kv_append_kernel(const AppendParams p) {
   st<T>(p.v_cache, vc, ld<T>(p.v_new, vn));
 }
 
-template <class T>
-__global__ __launch_bounds__(256) void rotary_q_kernel(const RotaryQParams p) {
-  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
+// Element idx of the query rotation; the keys of sequence b end `added` past
+// seqlens[b].
+template <class T, class F>
+__device__ inline void rotate_q_element(const RotaryQParams& p, int64_t idx, int added, F tables) {
   const int64_t total = (int64_t)p.batch * p.seqlen_q * p.heads * p.head_dim;
   if (idx >= total) return;
   const int d = (int)(idx % p.head_dim);
@@ -110,7 +124,7 @@ __global__ __launch_bounds__(256) void rotary_q_kernel(const RotaryQParams p) {
   r /= p.heads;
   const int i = (int)(r % p.seqlen_q);
   const int b = (int)(r / p.seqlen_q);
-  int64_t pos = (int64_t)p.seqlens[b] - p.seqlen_q + (p.leftpad != nullptr ? p.leftpad[b] : 0) + i;
+  int64_t pos = (int64_t)p.seqlens[b] + added - p.seqlen_q + (p.leftpad != nullptr ? p.leftpad[b] : 0) + i;
   // Negative positions count from the end of the tables (torch indexing in
   // the reference, flash_attn_interface.py:56).
   if (pos < 0) pos += p.table_rows;
@@ -122,12 +136,60 @@ __global__ __launch_bounds__(256) void rotary_q_kernel(const RotaryQParams p) {
     st<T>(p.out, oi, ld<T>(p.q, qi + d));
     return;
   }
-  const int half = p.rot >> 1;
-  st<T>(p.out, oi, rotate([&](int j) { return ld<T>(p.q, qi + j); }, d, p.cos + pos * half,
-                          p.sin + pos * half, p.rot, p.interleaved));
+  const auto t2 = tables(pos * (p.rot >> 1));
+  st<T>(p.out, oi, rotate([&](int j) { return ld<T>(p.q, qi + j); }, d, t2.c, t2.s, p.rot, p.interleaved));
+}
+
+struct F32Rows { const float* c; const float* s; };
+template <class T>
+struct TableRows { Table<T> c, s; };
+
+template <class T>
+__global__ __launch_bounds__(256) void kv_append_kernel(const AppendParams p) {
+  append_element<T>(p, (int64_t)blockIdx.x * 256 + threadIdx.x, p.cos != nullptr,
+                    [&](int64_t at) { return F32Rows{p.cos + at, p.sin + at}; });
+}
+
+template <class T>
+__global__ __launch_bounds__(256) void rotary_q_kernel(const RotaryQParams p) {
+  rotate_q_element<T>(p, (int64_t)blockIdx.x * 256 + threadIdx.x, 0,
+                      [&](int64_t at) { return F32Rows{p.cos + at, p.sin + at}; });
+}
+
+// Workgroups [0, n_append) append, the others rotate the queries; the first one
+// also writes the new lengths.  Bound by latency: a decode step moves a few
+// KiB, and the launches, table conversions and length sums it replaces (about
+// ten) were most of the call's host and GPU time.
+template <class T>
+__global__ __launch_bounds__(256) void kv_update_kernel(const UpdateParams p, int n_append) {
+  for (int i = 0; i < p.guard_n; ++i)
+    if (p.guard[i] != 0) return;   // a check failed: the cache stays as it is
+  if (p.lens_out != nullptr && blockIdx.x == 0)
+    for (int b = threadIdx.x; b < p.a.batch; b += 256) p.lens_out[b] = p.a.seqlens[b] + p.a.n_new;
+  auto tables = [&](int64_t at) {
+    return TableRows<T>{Table<T>{p.cos, p.table_dtype, at}, Table<T>{p.sin, p.table_dtype, at}};
+  };
+  if ((int)blockIdx.x < n_append)
+    append_element<T>(p.a, (int64_t)blockIdx.x * 256 + threadIdx.x, p.cos != nullptr, tables);
+  else if (p.cos != nullptr)
+    rotate_q_element<T>(p.q, (int64_t)(blockIdx.x - n_append) * 256 + threadIdx.x, p.a.n_new, tables);
 }
 
 }  // namespace fa
+
+hipError_t fa_launch_kv_update(int dtype, const fa::UpdateParams& p, hipStream_t st) {
+  const int64_t kv = (int64_t)p.a.batch * p.a.n_new * p.a.heads_k * p.a.head_dim;
+  const int64_t qn = p.cos != nullptr ? (int64_t)p.q.batch * p.q.seqlen_q * p.q.heads * p.q.head_dim : 0;
+  const int64_t nk = (kv + 255) / 256, nq = (qn + 255) / 256;
+  if (nk + nq <= 0) return hipSuccess;
+  if (nk + nq > 0x7fffffff) return hipErrorInvalidConfiguration;
+  const dim3 grid((unsigned)(nk + nq));
+  if (dtype == 0) hipLaunchKernelGGL(fa::kv_update_kernel<fa::F16>, grid, dim3(256), 0, st, p, (int)nk);
+  else if (dtype == 1) hipLaunchKernelGGL(fa::kv_update_kernel<fa::BF16>, grid, dim3(256), 0, st, p, (int)nk);
+  else hipLaunchKernelGGL(fa::kv_update_kernel<float>, grid, dim3(256), 0, st, p, (int)nk);
+  return hipGetLastError();
+}
+
 
 hipError_t fa_launch_kv_append(int dtype, const fa::AppendParams& p, hipStream_t st) {
   const int64_t total = (int64_t)p.batch * p.n_new * p.heads_k * p.head_dim;

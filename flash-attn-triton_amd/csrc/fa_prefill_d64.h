@@ -118,6 +118,7 @@ void prefill_d64_kernel(const FwdParams p) {
   table_ptr bt_row = nullptr;
   if constexpr (PAGED) bt_row = (table_ptr)(p.block_table + (int64_t)b * p.bt_stride);
   if constexpr (VARLEN) {
+    if (guard_failed(p)) return;
     const int qs = p.cu_q[b], ks = p.cu_k[b];
     Sq = p.cu_q[b + 1] - qs;
     Sk = p.cu_k[b + 1] - ks;

@@ -130,6 +130,7 @@ void prefill_kernel(const FwdParams p) {
 
   int Sq, Sk;
   int64_t q_base, o_base, lse_base, k_base, v_base;
+  if (guard_failed(p)) return;
   if (p.cu_q != nullptr) {
     const int qs = p.cu_q[b], ks = p.cu_k[b];
     Sq = p.cu_q[b + 1] - qs;

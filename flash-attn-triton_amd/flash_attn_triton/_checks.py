@@ -6,12 +6,14 @@ stream to drain (flash_attn_interface.py:433-470, :583-627).  ``Deferred``
 queues those checks and reads them all with one synchronization.  Range
 checks on device tensors (an array, an array plus an elementwise addend, or
 the differences of adjacent elements) reduce in one native launch per eight
-arrays (``fa_check_ranges``), which writes min and max straight into pinned
-host memory; other device scalars (flags, values) are packed by
-reinterpreting them as 32-bit words and copied with one device-to-host copy.
-A call whose launch is safe on unchecked arguments (``side=True``, the decode
-path) queues range checks only; they reduce on a second stream, so the launch
-does not queue behind them.  Exceptions keep the reference's order: a check
+distinct arrays (``fa_check_bounds``), which writes min and max straight into
+pinned host memory, where the host polls for them; other device scalars (flags,
+values) are packed by reinterpreting them as 32-bit words and copied with one
+device-to-host copy.  A call whose launch is safe on unchecked arguments
+(``side=True``, the decode path) queues range checks only; they reduce on a
+second stream, so the launch does not queue behind them.  A launch that is not
+can be guarded instead (``flush(launch, guarded=True)``): it takes the checks'
+device flags and does nothing when one is set.  Exceptions keep the reference's order: a check
 that fails on the host first raises the first failing device check queued
 before it, exactly as the reference's sequential checks would have.
 """
@@ -24,6 +26,7 @@ import torch
 
 from . import _native
 
+_I64_MIN, _I64_MAX = -(1 << 63), (1 << 63) - 1
 _WORDS = {torch.int32: 1, torch.float32: 1, torch.int64: 2, torch.float64: 2}
 
 
@@ -123,7 +126,12 @@ class Deferred:
         self.flush()
         raise exc
 
-    def flush(self, launch=None) -> list:
+    def ranges_only(self) -> bool:
+        """Whether only range checks of device arrays are queued (what a
+        guarded launch can be guarded with)."""
+        return all(it[0] == "range" and it[4][0].is_cuda for it in self._items)
+
+    def flush(self, launch=None, guarded: bool = False) -> list:
         """Raise the first failing queued check; return the queued values.
 
         With ``launch`` (a callable that enqueues kernels on the current
@@ -134,37 +142,54 @@ class Deferred:
         ``side=True`` the range checks reduce on a second stream, so the
         launch does not queue behind them.  Only kernels that stay inside
         their buffers whatever the checked arrays hold may be launched this
-        way."""
+        way, or, with ``guarded`` (``ranges_only()`` must hold), kernels that
+        return at once when one of the int32 device flags ``launch(flags)``
+        gets is set (None: nothing was checked on the device)."""
         items, self._items = self._items, []
         self._nvalues = 0
         if not items:
             if launch is not None:
-                launch()
+                launch(None) if guarded else launch()
             return []
-        # Range reductions: one fa_check_ranges launch per eight device
-        # arrays, results in pinned host memory; host tensors on the host.
+        # Range reductions: one launch per eight distinct device arrays (an
+        # array checked against several bounds reduces once), results in pinned
+        # host memory; host tensors on the host.
         ranged = [i for i, it in enumerate(items) if it[0] in ("range", "minmax")]
         on_dev = [i for i in ranged if items[i][4][0].is_cuda]
         results = {i: _host_minmax(*items[i][4]) for i in ranged if not items[i][4][0].is_cuda}
-        done = None
-        host_rng = None
+        done = host_rng = guard = handle = None
+        jobs, job_of = [], {}
         if on_dev:
-            device = items[on_dev[0]][4][0].device
+            seen = {}
+            for i in on_dev:
+                a, b, diff = items[i][4]
+                lo = _I64_MIN if items[i][2] is None else max(items[i][2], _I64_MIN)
+                hi = _I64_MAX if items[i][3] is None else min(items[i][3], _I64_MAX)
+                key = (a.data_ptr(), a.numel(), a.dtype, diff,
+                       None if b is None else (b.data_ptr(), b.dtype))
+                j = seen.get(key)
+                if j is None:
+                    seen[key] = j = len(jobs)
+                    jobs.append([a, b, diff, lo, hi])
+                else:
+                    jobs[j][3] = max(jobs[j][3], lo)
+                    jobs[j][4] = min(jobs[j][4], hi)
+                job_of[i] = j
+            device = jobs[0][0].device
             stream = torch.cuda.current_stream(device)
             if self._side:
                 side = _side_stream(device)
                 side.wait_stream(stream)
                 stream = side
-            host_rng = torch.empty(2 * len(on_dev), dtype=torch.int64, pin_memory=True)
+            handle = stream.cuda_stream
+            host_rng = torch.empty(3 * len(jobs), dtype=torch.int64, pin_memory=True)
+            if guarded:
+                guard = torch.empty(len(jobs), dtype=torch.int32, device=device)
             step = _native.MAX_RANGE_CHECKS
-            with torch.cuda.stream(stream):
-                for s0 in range(0, len(on_dev), step):
-                    chunk = on_dev[s0:s0 + step]
-                    _native.check_ranges([items[i][4][:2] for i in chunk],
-                                         host_rng[2 * s0:2 * (s0 + len(chunk))],
-                                         diff=[items[i][4][2] for i in chunk])
-                done = torch.cuda.Event()
-                done.record()
+            for s0 in range(0, len(jobs), step):
+                chunk = jobs[s0:s0 + step]
+                _native.check_bounds(chunk, host_rng[3 * s0:3 * (s0 + len(chunk))],
+                                     None if guard is None else guard[s0:s0 + len(chunk)], handle)
         # Flags and values: packed into 32-bit words, one copy.
         scal = [i for i, it in enumerate(items) if it[0] in ("flag", "value")]
         words, dtypes, host_sc = [], [], None
@@ -180,21 +205,29 @@ class Deferred:
             if packed.is_cuda:
                 host_sc = torch.empty(packed.shape, dtype=packed.dtype, pin_memory=True)
                 host_sc.copy_(packed, non_blocking=True)
-                done = torch.cuda.Event()   # same stream as the range launches
+                done = torch.cuda.Event()
                 done.record()
             else:
                 words = packed.tolist()
+        failed = None
         if launch is not None:
-            launch()
+            try:
+                launch(guard) if guarded else launch()
+            except Exception as exc:   # a failing check goes first
+                failed = exc
+        # Every tensor checked on the device is referenced by `items` until this
+        # wait: none returns to the caching allocator (whose next user could
+        # overwrite it on the current stream) while a check reads it, and the
+        # pinned results outlive the writes to them.
+        if host_rng is not None:
+            _native.check_wait(host_rng, len(jobs), handle)
         if done is not None:
-            # Every tensor checked on the device is referenced by `items` until
-            # this wait: none returns to the caching allocator (whose next user
-            # could overwrite it on the current stream) while a check reads it.
             done.synchronize()
         if host_rng is not None:
             got = host_rng.tolist()
-            for k, i in enumerate(on_dev):
-                results[i] = (got[2 * k], got[2 * k + 1])
+            for i in on_dev:
+                j = job_of[i]
+                results[i] = (got[3 * j], got[3 * j + 1])
         if host_sc is not None:
             words = host_sc.tolist()
         scalars_dec, pos = [], 0
@@ -217,4 +250,6 @@ class Deferred:
                     raise exc
                 if kind == "value":
                     values.append(got)
+        if failed is not None:
+            raise failed
         return values

@@ -50,6 +50,10 @@ _SIGNATURES = {
                              _i64, _i64p, _i64p, _i64p, _i64p, _i64p, _int, _f32, _int, _i64,
                              _i64, _f32, _vp, _i64, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64,
                              _f32, _u64, _vp]),
+    "fa_fwd_varlen_guarded": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64,
+                                     _i64, _i64, _i64p, _i64p, _i64p, _i64p, _i64p, _int, _f32,
+                                     _int, _i64, _i64, _f32, _vp, _i64, _vp, _vp, _vp, _vp, _i64,
+                                     _i64, _i64, _i64, _f32, _u64, _vp, _int, _vp]),
     "fa_bwd_dense": (_int, [_vp] * 10 + [_i64] * 6 + [_i64p] * 9 +
                      [_int, _f32, _int, _i64, _i64, _i64, _f32, _vp, _i64, _vp, _i64p, _vp,
                       _i64p, _f32, _u64, _vp]),
@@ -72,7 +76,13 @@ _SIGNATURES = {
                                  _i64p, _i64p, _i64p, _i64p, _int, _vp]),
     "fa_rotary_q": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _int, _i64, _i64, _i64,
                            _i64, _i64p, _i64p, _int, _vp]),
+    "fa_kvcache_update": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _i64, _vp,
+                                 _i64, _vp, _vp, _int, _i64, _i64, _int, _vp, _vp, _i64, _i64,
+                                 _vp, _i64, _i64, _i64, _i64, _i64p, _i64p, _i64p, _i64p, _i64p,
+                                 _i64p, _int, _vp, _int, _vp]),
     "fa_check_ranges": (_int, [_int, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "fa_check_bounds": (_int, [_int, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "fa_check_wait": (_int, [_vp, _int, _vp]),
     "fa_quant_k_int8": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64p, _vp]),
     "fa_fwd_int8": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64p, _i64p,
                            _i64p, _f32, _int, _i64, _i64, _vp]),
@@ -114,16 +124,21 @@ def _check(status: int, what: str) -> None:
         raise RuntimeError(f"{what} failed (status {status}): {msg}")
 
 
+_I64_ARRAY = [ctypes.c_int64 * n for n in range(8)]
+
+
 def _strides(values: Sequence[int]):
-    return (ctypes.c_int64 * len(values))(*[int(v) for v in values])
+    return _I64_ARRAY[len(values)](*values)
 
 
 def _ptr(t: Optional[torch.Tensor]):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
-def _stream(device: torch.device):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+def _stream(device: torch.device) -> int:
+    """Handle of the device's current stream (the raw query: a Stream object per
+    launch costs as much as the argument conversion)."""
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def dtype_code(dtype: torch.dtype) -> int:
@@ -236,9 +251,11 @@ def attn_probs(q, k, lse, probs, lse_out, cu_q, cu_k, max_seqlen_q: int, max_seq
 def fwd_varlen(q, k, v, out, lse, cu_q, cu_k, max_seqlen_q: int, max_seqlen_k: int,
                softmax_scale: float, causal: bool, window_left: int, window_right: int,
                softcap: float, alibi, seqused_q=None, seqused_k=None, cu_out=None,
-               block_table=None, dropout_p: float = 0.0, dropout_seed: int = 0) -> None:
+               block_table=None, dropout_p: float = 0.0, dropout_seed: int = 0,
+               guard=None) -> None:
     """q [Tq,Hq,D], k/v [Tk,Hk,D] (or paged [pages,page,Hk,D] with block_table);
-    cu_* int32 [batch+1]; lse [Tout,Hq] or None; see fa_fwd_varlen."""
+    cu_* int32 [batch+1]; lse [Tout,Hq] or None; guard None or the int32 flags
+    of check_bounds; see fa_fwd_varlen and fa_fwd_varlen_guarded."""
     lib = load()
     Hq, D = q.shape[1], q.shape[2]
     paged = block_table is not None
@@ -246,7 +263,7 @@ def fwd_varlen(q, k, v, out, lse, cu_q, cu_k, max_seqlen_q: int, max_seqlen_k: i
     nkv = 3 if paged else 2
     batch = cu_q.numel() - 1
     lse_stride = _strides(lse.stride()) if lse is not None else None
-    status = lib.fa_fwd_varlen(
+    status = lib.fa_fwd_varlen_guarded(
         _ptr(q), _ptr(k), _ptr(v), _ptr(out), _ptr(lse), _ptr(cu_q), _ptr(cu_k), batch,
         int(max_seqlen_q), int(max_seqlen_k), Hq, Hk, D, _strides(q.stride()[:2]),
         _strides(k.stride()[:nkv]), _strides(v.stride()[:nkv]), _strides(out.stride()[:2]),
@@ -256,7 +273,7 @@ def fwd_varlen(q, k, v, out, lse, cu_q, cu_k, max_seqlen_q: int, max_seqlen_k: i
         _ptr(cu_out), _ptr(block_table), int(block_table.stride(0)) if paged else 0,
         int(k.shape[1]) if paged else 0, int(k.shape[0]) if paged else 0,
         int(block_table.shape[1]) if paged else 0, float(dropout_p), int(dropout_seed),
-        _stream(q.device))
+        _ptr(guard), 0 if guard is None else guard.numel(), _stream(q.device))
     _check(status, "fa_fwd_varlen")
 
 
@@ -383,6 +400,54 @@ def check_ranges(arrays, minmax, diff=None) -> None:
     status = lib.fa_check_ranges(n, ptr_a, bytes_a, ptr_b, bytes_b, diffs, numel,
                                  ctypes.c_void_p(minmax.data_ptr()), _stream(device))
     _check(status, "fa_check_ranges")
+
+
+def check_bounds(jobs, result, guard, stream: int) -> None:
+    """Range checks of ``jobs`` = [(a, b or None, diff, lo, hi), ...] (as
+    ``check_ranges``, at most MAX_RANGE_CHECKS; lo / hi int64 bounds) in one
+    launch on the stream handle ``stream``: min, max and a done mark per job
+    into ``result`` (pinned int64, 3 per job), the outcome into ``guard`` (int32
+    device flags, one per job, or None).  See fa_check_bounds."""
+    n = len(jobs)
+    a, b, diff, lo, hi = zip(*jobs)
+    status = load().fa_check_bounds(
+        n, (ctypes.c_void_p * n)(*[t.data_ptr() for t in a]),
+        (ctypes.c_int * n)(*[t.element_size() for t in a]),
+        (ctypes.c_void_p * n)(*[None if t is None else t.data_ptr() for t in b]),
+        (ctypes.c_int * n)(*[4 if t is None else t.element_size() for t in b]),
+        (ctypes.c_int * n)(*diff), (ctypes.c_int64 * n)(*[t.numel() for t in a]),
+        (ctypes.c_int64 * n)(*lo), (ctypes.c_int64 * n)(*hi),
+        ctypes.c_void_p(result.data_ptr()), _ptr(guard), ctypes.c_void_p(stream))
+    _check(status, "fa_check_bounds")
+
+
+def check_wait(result, n: int, stream: int) -> None:
+    """Wait until the n results of ``check_bounds`` launches on ``stream`` are written."""
+    _check(load().fa_check_wait(ctypes.c_void_p(result.data_ptr()), n, ctypes.c_void_p(stream)),
+           "fa_check_wait")
+
+
+def kvcache_update(k_new, v_new, k_cache, v_cache, cache_seqlens, block_table, cache_batch_idx,
+                   cache_leftpad, capacity: int, rotary_cos, rotary_sin, rotary_interleaved: bool,
+                   q, q_out, lens_out, guard) -> None:
+    """Append k_new / v_new [B, n, Hk, D] (None: nothing) in place and rotate q
+    into q_out (rotary_cos / sin given) in one launch (see fa_kvcache_update)."""
+    n, heads_k = (0, k_cache.shape[2]) if k_new is None else k_new.shape[1:3]
+    paged = block_table is not None
+    rotary = rotary_cos is not None
+    B, Sq, Hq, D = q.shape
+    st = [None if t is None else _strides(t.stride()[:3])
+          for t in (k_new, v_new, k_cache, v_cache, q, q_out)]
+    status = load().fa_kvcache_update(
+        _ptr(k_new), _ptr(v_new), _ptr(k_cache), _ptr(v_cache), _ptr(cache_seqlens),
+        _ptr(block_table), block_table.stride(0) if paged else 0, k_cache.shape[1] if paged else 0,
+        k_cache.shape[0] if paged else 0, _ptr(cache_batch_idx), 0 if paged else k_cache.shape[0],
+        _ptr(cache_leftpad), int(capacity), _ptr(rotary_cos), _ptr(rotary_sin),
+        dtype_code(rotary_cos.dtype) if rotary else 0, 2 * rotary_cos.shape[-1] if rotary else 0,
+        rotary_cos.shape[0] if rotary else 0, int(bool(rotary_interleaved)), _ptr(q), _ptr(q_out),
+        Sq, Hq, _ptr(lens_out), B, n, heads_k, D, *st, dtype_code(q.dtype), _ptr(guard),
+        0 if guard is None else guard.numel(), _stream(q.device))
+    _check(status, "fa_kvcache_update")
 
 
 def quant_k_int8(k, k8, s_k) -> None:

@@ -53,6 +53,7 @@ from . import _native
 from ._checks import Deferred
 
 BLOCK_SIZE = 64
+_TABLE_DTYPES = (torch.float16, torch.bfloat16, torch.float32)
 
 def _normalize_alibi(alibi_slopes, batch, heads, device):
     """(H,) or (B,H) fp32 slopes -> contiguous (B,H) (flash_attn_interface.py:128-136)."""
@@ -323,6 +324,23 @@ def flash_attn_kvpacked_func(q, kv, dropout_p=0.0, softmax_scale=None, causal=Fa
                            attn_bias)
 
 
+def _outlasts_the_host(q, k_cache, block_table) -> bool:
+    """Whether the attention launch of a KV-cache call with full caches would
+    run longer than the host takes for the call (about 60 us).  Then the checks
+    go to a second stream: making it wait for the caller's costs the host 16 us,
+    which the GPU's work hides, and the launch does not queue behind them.
+    Otherwise the host is the bound and the checks (4 us on the GPU) go ahead of
+    the launch on its own stream.  Rates: 5 TB/s, 0.8 PFLOP/s."""
+    if q.ndim != 4 or k_cache.ndim != 4:
+        return False
+    keys = k_cache.shape[0] * k_cache.shape[1]
+    if block_table is not None and block_table.ndim == 2:
+        keys = block_table.shape[0] * block_table.shape[1] * k_cache.shape[1]
+    nbytes = 2 * keys * k_cache.shape[2] * k_cache.shape[3] * k_cache.element_size()
+    flops = 4 * keys * q.shape[1] * q.shape[2] * q.shape[3]
+    return max(nbytes / 5e12, flops / 8e14) > 60e-6
+
+
 def flash_attn_with_kvcache(
     q,
     k_cache,
@@ -351,14 +369,16 @@ def flash_attn_with_kvcache(
     Returns (batch, seqlen_q, nheads, headdim).
     """
     paged = block_table is not None
-    # Without an append, rotary or ALiBi slopes nothing the launch needs comes
-    # from the device checks, and the kernels keep every read inside the
-    # caches and the block table whatever cache_seqlens and block_table hold
-    # (fa_fwd_kvcache clamps them): the checks then run on a second stream
-    # and the attention launch goes out before the host waits for them; they
-    # still raise before this call returns.
-    launch_first = k is None and v is None and rotary_cos is None and alibi_slopes is None
-    chk = Deferred(side=launch_first)
+    # Without ALiBi slopes or gradients nothing the launches need comes from the
+    # device checks, and the kernels keep every read inside the caches and the
+    # block table whatever cache_seqlens and block_table hold (fa_fwd_kvcache
+    # clamps them): the launches then go out before the host waits for the
+    # checks, which still raise before this call returns.  An append, which
+    # writes the cache, is guarded by the checks' device flags on the same
+    # stream; a long attention launch has its checks on a second stream.
+    launch_first = alibi_slopes is None and not _needs_grad(q, k_cache, v_cache)
+    chk = Deferred(side=launch_first and k is None and v is None
+                   and _outlasts_the_host(q, k_cache, block_table))
     if (rotary_cos is None) != (rotary_sin is None):
         raise ValueError("rotary_cos and rotary_sin must be supplied together")
     if q.ndim != 4 or k_cache.ndim != 4 or v_cache.ndim != 4:
@@ -402,7 +422,6 @@ def flash_attn_with_kvcache(
         if leftpads.numel() != q.shape[0]:
             chk.fail(bad_pads)
         chk.check_range(leftpads, 0, None, bad_pads)
-    zero_pad = 0 if leftpads is None else leftpads
     cos_t = sin_t = None
     if rotary_cos is not None:
         # The reference casts the tables to the input dtype before rotating
@@ -412,8 +431,13 @@ def flash_attn_with_kvcache(
                                 "tables of the same shape"))
         if rotary_cos.shape[-1] * 2 > q.shape[-1]:
             chk.fail(ValueError("rotary tables exceed the head dimension"))
-        cos_t = rotary_cos.to(device=q.device).to(q.dtype).float().contiguous()
-        sin_t = rotary_sin.to(device=q.device).to(q.dtype).float().contiguous()
+        if launch_first and rotary_cos.dtype == rotary_sin.dtype and rotary_cos.dtype in _TABLE_DTYPES:
+            # fa_kvcache_update rounds the tables as it reads them.
+            cos_t = rotary_cos.to(device=q.device).contiguous()
+            sin_t = rotary_sin.to(device=q.device).contiguous()
+        else:
+            cos_t = rotary_cos.to(device=q.device).to(q.dtype).float().contiguous()
+            sin_t = rotary_sin.to(device=q.device).to(q.dtype).float().contiguous()
     bad_rotary = IndexError("rotary position out of range of the cos/sin tables")
     n_new = 0
     if k is not None or v is not None:
@@ -431,9 +455,9 @@ def flash_attn_with_kvcache(
         if lengths.numel() != q.shape[0]:
             chk.fail(bad_fit)
         chk.check_range(lengths, 0, None, bad_fit)
-        chk.check_range(lengths + zero_pad + n_new, None, cache_capacity, bad_fit)
-        if cos_t is not None and lengths.numel() and n_new:
-            chk.check((lengths + zero_pad + n_new > cos_t.shape[0]).any(), bad_rotary)
+        chk.check_range(lengths, None, cache_capacity - n_new, bad_fit, plus=leftpads)
+        if cos_t is not None and n_new:
+            chk.check_range(lengths, None, cos_t.shape[0] - n_new, bad_rotary, plus=leftpads)
     else:
         if cache_seqlens is None:
             lengths = torch.full((q.shape[0],), cache_capacity, dtype=torch.int32, device=q.device)
@@ -450,13 +474,12 @@ def flash_attn_with_kvcache(
         else:
             chk.check_range(lengths, 0, None, bad_lengths)
             chk.check_range(lengths, None, cache_capacity, bad_lengths, plus=leftpads)
-    if cos_t is not None and lengths.numel() and q.shape[1]:
+    if cos_t is not None and q.shape[1]:
         # Query rows rotate at L + leftpad - Sq + i (L after the append);
         # negative positions index from the end of the tables, as torch
         # indexing does in the reference (:516-517).
-        first = lengths + n_new + zero_pad - q.shape[1]
-        chk.check((first + q.shape[1] > cos_t.shape[0]).any() | (first < -cos_t.shape[0]).any(),
-                  bad_rotary)
+        chk.check_range(lengths, q.shape[1] - n_new - cos_t.shape[0], cos_t.shape[0] - n_new,
+                        bad_rotary, plus=leftpads)
     if q.shape[-1] not in (16, 32, 64, 128, 256):
         chk.fail(ValueError("head dimension must be one of 16, 32, 64, 128, or 256"))
     if q.shape[2] % k_cache.shape[2] != 0:
@@ -480,34 +503,43 @@ def flash_attn_with_kvcache(
     bt32 = block_table.to(device=q.device, dtype=torch.int32).contiguous() if paged else None
     rows32 = cache_rows.to(torch.int32).contiguous() if cache_rows is not None else None
     pads32 = leftpads.to(torch.int32).contiguous() if leftpads is not None else None
+    kn = vn = None
     if n_new:
         kn = k.to(device=q.device, dtype=k_cache.dtype)
         vn = v.to(device=q.device, dtype=v_cache.dtype)
-        _native.kvcache_append(kn, vn, k_cache, v_cache, lengths32, bt32, rows32, pads32,
-                               int(cache_capacity), cos_t, sin_t, rotary_interleaved)
-        lengths32 = (lengths32 + n_new).to(torch.int32)
-    if _needs_grad(q, k_cache, v_cache):
-        if launch_first:
-            chk.flush()
-        return _kvcache_differentiable(q, k_cache, v_cache, lengths32, bt32, cache_rows, pads32,
-                                       cos_t, sin_t, rotary_interleaved, softmax_scale, causal,
-                                       window_size, alibi)
+    if not launch_first:
+        if n_new:
+            _native.kvcache_append(kn, vn, k_cache, v_cache, lengths32, bt32, rows32, pads32,
+                                   int(cache_capacity), cos_t, sin_t, rotary_interleaved)
+            lengths32 = (lengths32 + n_new).to(torch.int32)
+        if _needs_grad(q, k_cache, v_cache):
+            return _kvcache_differentiable(q, k_cache, v_cache, lengths32, bt32, cache_rows,
+                                           pads32, cos_t, sin_t, rotary_interleaved,
+                                           softmax_scale, causal, window_size, alibi)
     qk = _kernel_ready(q)
-    if cos_t is not None and q.shape[1]:
-        q_rot = torch.empty(q.shape, dtype=q.dtype, device=q.device)
-        _native.rotary_q(q, q_rot, lengths32, pads32, cos_t, sin_t, rotary_interleaved)
-        qk = q_rot
-    kc, vc = _kernel_ready(k_cache), _kernel_ready(v_cache)
+    rotate = cos_t is not None and q.shape[1] > 0
+    if rotate:
+        qk = torch.empty(q.shape, dtype=q.dtype, device=q.device)
+        if not launch_first:
+            _native.rotary_q(q, qk, lengths32, pads32, cos_t, sin_t, rotary_interleaved)
     out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
 
-    def launch():
+    def launch(guard=None):
+        lens = lengths32
+        if launch_first and (n_new or rotate):
+            if n_new:
+                lens = torch.empty_like(lengths32)
+            _native.kvcache_update(kn, vn, k_cache, v_cache, lengths32, bt32, rows32, pads32,
+                                   int(cache_capacity), cos_t, sin_t, rotary_interleaved, q,
+                                   qk if rotate else None, lens if n_new else None, guard)
+        # (A cache that the kernels cannot read in place is copied after the append.)
         _native.fwd_kvcache(
-            qk, kc, vc, out, None, lengths32,
-            bt32, rows32, pads32,
-            int(cache_capacity), softmax_scale, causal, window_size[0], window_size[1], alibi)
+            qk, _kernel_ready(k_cache), _kernel_ready(v_cache), out, None, lens, bt32, rows32,
+            pads32, int(cache_capacity), softmax_scale, causal, window_size[0], window_size[1],
+            alibi)
 
     if launch_first:
-        chk.flush(launch)   # the one host synchronization of this call
+        chk.flush(launch, guarded=n_new > 0)   # the one host synchronization of this call
     else:
         launch()
     return _wrap_grad(out, q)
@@ -772,6 +804,19 @@ def flash_attn_varlen_func(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q,
         return _varlen_attention_with_probs(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q,
                                             max_seqlen_k, dropout_p, softmax_scale, causal,
                                             window_size, softcap, alibi)
+    plain = not (paged or seqused_q is not None or seqused_k is not None)
+    if plain and alibi is None and chk.ranges_only():
+        # Nothing below depends on a checked value: the launch goes out first,
+        # guarded by the checks' device flags, and the host waits for the checks
+        # (the one synchronization of this call) while it runs.
+        seed = new_dropout_seed() if dropout_p > 0.0 else 0
+        scale = 1.0 / math.sqrt(q.shape[-1]) if softmax_scale is None else softmax_scale
+        result = []
+        chk.flush(lambda guard: result.append(varlen_attention(
+            q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, softmax_scale=scale,
+            causal=causal, window_left=window_size[0], window_right=window_size[1],
+            softcap=softcap, dropout_p=dropout_p, dropout_seed=seed, guard=guard)), guarded=True)
+        return result[0]
     values = chk.flush()   # the one host synchronization of this call
     seed = new_dropout_seed() if dropout_p > 0.0 else 0
     use_alibi = alibi is not None and values[alibi_bits] != (0, 0)

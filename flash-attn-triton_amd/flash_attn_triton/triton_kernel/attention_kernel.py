@@ -67,11 +67,12 @@ def _kernel_ready(t: torch.Tensor) -> torch.Tensor:
     that are multiples of 16 bytes and a 16-byte aligned base.  Other layouts
     get one contiguous copy (the reference copies every non-contiguous input,
     flash_attn_interface.py:202-204)."""
+    strides = t.stride()
+    low = t.data_ptr()
     es = t.element_size()
-    if (t.stride(-1) == 1 and all((s * es) % 16 == 0 for s in t.stride()[:-1])
-            and t.data_ptr() % 16 == 0):
-        return t
-    return t.contiguous()
+    for s in strides[:-1]:
+        low |= s * es
+    return t if strides[-1] == 1 and low % 16 == 0 else t.contiguous()
 
 
 def dense_forward(q, k, v, *, softmax_scale: float, causal: bool, q_pos_offset: int = 0,
@@ -105,13 +106,14 @@ def varlen_forward(q, k, v, cu_q, cu_k, max_seqlen_q: int, max_seqlen_k: int, *,
                    seqused_k: Optional[torch.Tensor] = None,
                    out_rows: Optional[int] = None, cu_out: Optional[torch.Tensor] = None,
                    block_table: Optional[torch.Tensor] = None, dropout_p: float = 0.0,
-                   dropout_seed: int = 0):
+                   dropout_seed: int = 0, guard: Optional[torch.Tensor] = None):
     """Run the packed varlen HIP kernel on ``[T, H, D]`` tensors.
 
     ``seqused_q``/``seqused_k`` limit each sequence to its first queries /
     keys; with ``cu_out`` the outputs of the used queries are packed into
     ``out_rows`` rows (sequence b at ``cu_out[b]``).  With ``block_table``
-    k / v are paged caches ``[pages, page_size, Hk, D]``."""
+    k / v are paged caches ``[pages, page_size, Hk, D]``.  ``guard``: device
+    flags of argument checks still in flight (``Deferred.flush``)."""
     dev = q.device
     qk, kk, vk = _kernel_ready(q), _kernel_ready(k), _kernel_ready(v)
     rows = q.shape[0] if out_rows is None else int(out_rows)
@@ -127,7 +129,7 @@ def varlen_forward(q, k, v, cu_q, cu_k, max_seqlen_q: int, max_seqlen_k: int, *,
     _native.fwd_varlen(qk, kk, vk, out, lse, i32(cu_q), i32(cu_k), max_seqlen_q, max_seqlen_k,
                        softmax_scale, causal, window_left, window_right, softcap, alibi,
                        i32(seqused_q), i32(seqused_k), i32(cu_out), i32(block_table),
-                       dropout_p, dropout_seed)
+                       dropout_p, dropout_seed, guard)
     return (out, lse) if return_lse else out
 
 
@@ -252,12 +254,12 @@ class _VarlenAttention(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, q, k, v, cu_q, cu_k, max_seqlen_q, max_seqlen_k, softmax_scale, causal,
-                window_left, window_right, softcap, alibi, dropout_p, dropout_seed):
+                window_left, window_right, softcap, alibi, dropout_p, dropout_seed, guard):
         out, lse = varlen_forward(q, k, v, cu_q, cu_k, max_seqlen_q, max_seqlen_k,
                                   softmax_scale=softmax_scale, causal=causal,
                                   window_left=window_left, window_right=window_right,
                                   softcap=softcap, alibi=alibi, return_lse=True,
-                                  dropout_p=dropout_p, dropout_seed=dropout_seed)
+                                  dropout_p=dropout_p, dropout_seed=dropout_seed, guard=guard)
         ctx.save_for_backward(q, k, v, out, lse, cu_q, cu_k, alibi)
         ctx.opts = (max_seqlen_q, max_seqlen_k, softmax_scale, causal, window_left,
                     window_right, softcap, dropout_p, dropout_seed)
@@ -272,7 +274,7 @@ class _VarlenAttention(torch.autograd.Function):
                                      softmax_scale=scale, causal=causal, window_left=wl,
                                      window_right=wr, softcap=cap, alibi=alibi, dropout_p=dp,
                                      dropout_seed=seed)
-        return (dq, dk, dv) + (None,) * 12
+        return (dq, dk, dv) + (None,) * 13
 
 
 def dense_attention(q, k, v, *, softmax_scale: float, causal: bool, q_pos_offset: int = 0,
@@ -300,17 +302,18 @@ def varlen_attention(q, k, v, cu_q, cu_k, max_seqlen_q: int, max_seqlen_k: int, 
                      softmax_scale: float, causal: bool, window_left: int = -1,
                      window_right: int = -1, softcap: float = 0.0,
                      alibi: Optional[torch.Tensor] = None, return_lse: bool = False,
-                     dropout_p: float = 0.0, dropout_seed: int = 0):
+                     dropout_p: float = 0.0, dropout_seed: int = 0,
+                     guard: Optional[torch.Tensor] = None):
     """``varlen_forward`` that is differentiable in q, k, v (fp16 / bf16)."""
     if not _needs_grad(q, k, v):
         return varlen_forward(q, k, v, cu_q, cu_k, max_seqlen_q, max_seqlen_k,
                               softmax_scale=softmax_scale, causal=causal,
                               window_left=window_left, window_right=window_right,
                               softcap=softcap, alibi=alibi, return_lse=return_lse,
-                              dropout_p=dropout_p, dropout_seed=dropout_seed)
+                              dropout_p=dropout_p, dropout_seed=dropout_seed, guard=guard)
     out, lse = _VarlenAttention.apply(q, k, v, cu_q, cu_k, max_seqlen_q, max_seqlen_k,
                                       softmax_scale, causal, window_left, window_right, softcap,
-                                      alibi, dropout_p, dropout_seed)
+                                      alibi, dropout_p, dropout_seed, guard)
     return (out, lse) if return_lse else out
 
 

@@ -128,6 +128,24 @@ int fa_fwd_varlen(const void* q, const void* k, const void* v, void* out, float*
                   int64_t num_pages, int64_t block_table_cols, float dropout_p,
                   uint64_t dropout_seed, fa_stream_t stream);
 
+/* fa_fwd_varlen for a launch issued before the host has read the checks of its
+ * device arguments: guard (device, guard_n words, as fa_check_bounds writes
+ * them) is read first, and when any word is nonzero the kernel returns without
+ * reading cu_seqlens or writing anything. */
+int fa_fwd_varlen_guarded(const void* q, const void* k, const void* v, void* out, float* lse,
+                  const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, int64_t batch,
+                  int64_t max_seqlen_q, int64_t max_seqlen_k, int64_t heads_q, int64_t heads_k,
+                  int64_t head_dim, const int64_t* q_stride, const int64_t* k_stride,
+                  const int64_t* v_stride, const int64_t* o_stride, const int64_t* lse_stride,
+                  int dtype, float softmax_scale, int causal, int64_t window_left,
+                  int64_t window_right, float softcap, const float* alibi_slopes,
+                  int64_t alibi_batch_stride, const int32_t* seqused_q,
+                  const int32_t* seqused_k, const int32_t* cu_seqlens_out,
+                  const int32_t* block_table, int64_t block_table_stride, int64_t page_size,
+                  int64_t num_pages, int64_t block_table_cols, float dropout_p,
+                  uint64_t dropout_seed, const int32_t* guard, int guard_n,
+                  fa_stream_t stream);
+
 /* Backward of fa_fwd_dense: dq, dk, dv from dout.
  *
  * Replaces `_dense_backward` (attention_kernel.py:1104-1155: the
@@ -327,6 +345,27 @@ int fa_rotary_q(const void* q, void* out, const int32_t* cache_seqlens,
                 int64_t seqlen_q, int64_t heads, int64_t head_dim, const int64_t* q_stride,
                 const int64_t* out_stride, int dtype, fa_stream_t stream);
 
+/* The append of fa_kvcache_append and the query rotation of fa_rotary_q in one
+ * launch: n_new may be 0 (no append) and rotary_cos NULL (no rotation).  The
+ * tables are [rotary_rows, rotary_dim / 2] contiguous of table_dtype, rounded
+ * to `dtype` as they are read.  cache_seqlens holds the lengths before the
+ * append; lens_out (nullable, int32 [batch]) receives them plus n_new, and the
+ * queries are rotated at those.  With a failed guard (see fa_check_bounds)
+ * nothing is written. */
+int fa_kvcache_update(const void* k_new, const void* v_new, void* k_cache, void* v_cache,
+                      const int32_t* cache_seqlens, const int32_t* block_table,
+                      int64_t block_table_stride, int64_t page_size, int64_t num_pages,
+                      const int32_t* cache_batch_idx, int64_t cache_rows,
+                      const int32_t* cache_leftpad, int64_t capacity, const void* rotary_cos,
+                      const void* rotary_sin, int table_dtype, int64_t rotary_dim,
+                      int64_t rotary_rows, int rotary_interleaved, const void* q, void* q_out,
+                      int64_t seqlen_q, int64_t heads_q, int32_t* lens_out, int64_t batch,
+                      int64_t n_new, int64_t heads_k, int64_t head_dim,
+                      const int64_t* k_new_stride, const int64_t* v_new_stride,
+                      const int64_t* k_cache_stride, const int64_t* v_cache_stride,
+                      const int64_t* q_stride, const int64_t* q_out_stride, int dtype,
+                      const int32_t* guard, int guard_n, fa_stream_t stream);
+
 /* Range checks of integer device arrays in one launch: the validation of the
  * KV-cache call's device arguments (replaces the `torch.any(...)` / `.item()`
  * chain of flash_attn_interface.py:428-453 that checks the block table,
@@ -346,6 +385,20 @@ int fa_rotary_q(const void* q, void* out, const int32_t* cache_seqlens,
 int fa_check_ranges(int n, const void* const* a, const int* a_bytes, const void* const* b,
                     const int* b_bytes, const int* diff, const int64_t* numel, int64_t* minmax,
                     fa_stream_t stream);
+
+/* fa_check_ranges with bounds and a result the host can poll.  result is
+ * pinned host memory, 3 int64 per array: min, max and a mark that becomes
+ * nonzero once both are written (the call clears it first).  guard (nullable)
+ * is device memory, one word per array: 1 if min < lo[i] or max > hi[i], else
+ * 0, for launches on the same stream to be guarded with.  Rejected on a
+ * capturing stream. */
+int fa_check_bounds(int n, const void* const* a, const int* a_bytes, const void* const* b,
+                    const int* b_bytes, const int* diff, const int64_t* numel, const int64_t* lo,
+                    const int64_t* hi, int64_t* result, int32_t* guard, fa_stream_t stream);
+
+/* Waits until the n results of fa_check_bounds launches on `stream` are
+ * written.  Fails if the stream fails, or drains without them. */
+int fa_check_wait(const int64_t* result, int n, fa_stream_t stream);
 
 /* Per-token INT8 quantization of K (fp16), bit-exact with
  * `_quantize_k_rows` (attention_kernel_int8.py:58-79, launched at :232):
