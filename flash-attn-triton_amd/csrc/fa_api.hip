@@ -451,7 +451,7 @@ int fa_bwd_dense(const void* q, const void* k, const void* v, const void* out, c
                     dropout_seed, (hipStream_t)stream);
 }
 
-int fa_bwd_varlen(const void* q, const void* k, const void* v, const void* out,
+int fa_bwd_varlen_sized(const void* q, const void* k, const void* v, const void* out,
                   const void* dout, const float* lse, void* dq, void* dk, void* dv, float* delta,
                   const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, int64_t batch,
                   int64_t max_seqlen_q, int64_t max_seqlen_k, int64_t heads_q, int64_t heads_k,
@@ -461,7 +461,7 @@ int fa_bwd_varlen(const void* q, const void* k, const void* v, const void* out,
                   const int64_t* lse_stride, int dtype, float softmax_scale, int causal,
                   int64_t window_left, int64_t window_right, float softcap,
                   const float* alibi_slopes, int64_t alibi_batch_stride, float dropout_p,
-                  uint64_t dropout_seed, fa_stream_t stream) {
+                  uint64_t dropout_seed, int64_t total_k, fa_stream_t stream) {
   const char* name = "fa_bwd_varlen";
   int rc = bwd_check_common(name, q, k, v, out, dout, lse, dq, dk, dv, delta, dtype, head_dim,
                             heads_q, heads_k);
@@ -492,11 +492,36 @@ int fa_bwd_varlen(const void* q, const void* k, const void* v, const void* out,
   p.dv_ss = dv_stride[0]; p.dv_sh = dv_stride[1];
   p.lse_ss = lse_stride[0]; p.lse_sh = lse_stride[1];
   p.cu_q = cu_seqlens_q; p.cu_k = cu_seqlens_k;
+  p.total_k = total_k;
   p.batch = (int)batch; p.seqlen_q = (int)max_seqlen_q; p.seqlen_k = (int)max_seqlen_k;
   p.heads_q = (int)heads_q; p.heads_k = (int)heads_k; p.group = (int)(heads_q / heads_k);
   return bwd_launch(name, p, dtype, head_dim, softmax_scale, softcap, alibi_slopes,
                     alibi_batch_stride, causal, window_left, window_right, dropout_p,
                     dropout_seed, (hipStream_t)stream);
+}
+
+int fa_bwd_varlen(const void* q, const void* k, const void* v, const void* out,
+                  const void* dout, const float* lse, void* dq, void* dk, void* dv, float* delta,
+                  const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, int64_t batch,
+                  int64_t max_seqlen_q, int64_t max_seqlen_k, int64_t heads_q, int64_t heads_k,
+                  int64_t head_dim, const int64_t* q_stride, const int64_t* k_stride,
+                  const int64_t* v_stride, const int64_t* o_stride, const int64_t* do_stride,
+                  const int64_t* dq_stride, const int64_t* dk_stride, const int64_t* dv_stride,
+                  const int64_t* lse_stride, int dtype, float softmax_scale, int causal,
+                  int64_t window_left, int64_t window_right, float softcap,
+                  const float* alibi_slopes, int64_t alibi_batch_stride, float dropout_p,
+                  uint64_t dropout_seed, fa_stream_t stream) {
+  return fa_bwd_varlen_sized(q, k, v, out, dout, lse, dq, dk, dv, delta, cu_seqlens_q,
+                             cu_seqlens_k, batch, max_seqlen_q,
+                             max_seqlen_k, heads_q, heads_k,
+                             head_dim, q_stride, k_stride,
+                             v_stride, o_stride, do_stride,
+                             dq_stride, dk_stride, dv_stride,
+                             lse_stride, dtype, softmax_scale,
+                             causal, window_left, window_right,
+                             softcap, alibi_slopes,
+                             alibi_batch_stride, dropout_p,
+                             dropout_seed, 0, stream);
 }
 
 int fa_fwd_kvcache_plan(int64_t batch, int64_t seqlen_q, int64_t heads_q, int64_t heads_k,

@@ -33,6 +33,7 @@ struct BwdParams {
   int causal, window_left, window_right;
   int64_t q_offset;                               // query row i sits at position i + q_offset
   const int* cu_q; const int* cu_k;
+  int64_t total_k;                                // varlen: packed keys (0: unknown)
   DropoutCfg drop;                                // the forward's dropout (GENERIC only)
   // Optional fp32 additive bias of the dense forward (after ALiBi, before
   // softcap), bias[b*bias_sb + h*bias_sh + i*bias_sq + j*bias_sk], and the
@@ -41,7 +42,7 @@ struct BwdParams {
   // gradients sum).
   const float* bias; int64_t bias_sb, bias_sh, bias_sq, bias_sk;
   float* dbias; int64_t dbias_sb, dbias_sh, dbias_sq, dbias_sk;
-  int n_blocks, total_blocks;                     // filled by the launcher
+  int n_blocks, total_blocks, span;               // filled by the launcher (span: work_item's)
 };
 
 }  // namespace fa

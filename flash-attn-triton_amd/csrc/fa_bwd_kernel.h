@@ -174,18 +174,20 @@ void bwd_dq_kernel(const BwdParams p) {
   // unevenly).
   int mb, id;
   if (!VARLEN ||
-      !work_item_kv_rr(blockIdx.x, p.total_blocks, p.n_blocks, p.group, p.causal != 0, mb, id))
-    work_item(blockIdx.x, p.total_blocks, p.n_blocks, p.causal != 0, kBwdCausalSpan, mb, id);
+      !work_item_kv_rr(blockIdx.x, p.total_blocks, p.n_blocks, p.group, p.causal != 0, p.span, mb, id))
+    work_item(blockIdx.x, p.total_blocks, p.n_blocks, p.causal != 0, p.span, mb, id);
   const int hh = id % p.heads_q;
-  const int b = id / p.heads_q;
+  int b = id / p.heads_q;
   const int kvh = hh / p.group;
 
   int Sq = p.seqlen_q, Sk = p.seqlen_k, qs = 0, ks = 0;
-  if (p.cu_q != nullptr) {
-    qs = p.cu_q[b];
-    ks = p.cu_k[b];
-    Sq = p.cu_q[b + 1] - qs;
-    Sk = p.cu_k[b + 1] - ks;
+  if constexpr (VARLEN) {
+    const VarlenSeq sq = nth_longest(p.cu_q, p.cu_k, p.batch, b);
+    b = sq.b;
+    qs = sq.qs;
+    ks = sq.ks;
+    Sq = sq.Sq;
+    Sk = sq.Sk;
   }
   const int row0 = mb * BM;
   if (row0 >= Sq) return;
@@ -568,18 +570,20 @@ void bwd_dkdv_kernel(const BwdParams p) {
   // heads round-robin over the XCDs.
   int nb, id;
   if (!VARLEN ||
-      !work_item_kv_rr(blockIdx.x, p.total_blocks, p.n_blocks, 1, p.causal != 0, nb, id))
-    work_item(blockIdx.x, p.total_blocks, p.n_blocks, p.causal != 0, kBwdCausalSpan, nb, id);
+      !work_item_kv_rr(blockIdx.x, p.total_blocks, p.n_blocks, 1, p.causal != 0, p.span, nb, id))
+    work_item(blockIdx.x, p.total_blocks, p.n_blocks, p.causal != 0, p.span, nb, id);
   if (p.causal) nb = p.n_blocks - 1 - nb;
   const int kvh = id % p.heads_k;
-  const int b = id / p.heads_k;
+  int b = id / p.heads_k;
 
   int Sq = p.seqlen_q, Sk = p.seqlen_k, qs = 0, ks = 0;
-  if (p.cu_q != nullptr) {
-    qs = p.cu_q[b];
-    ks = p.cu_k[b];
-    Sq = p.cu_q[b + 1] - qs;
-    Sk = p.cu_k[b + 1] - ks;
+  if constexpr (VARLEN) {
+    const VarlenSeq sq = nth_longest(p.cu_q, p.cu_k, p.batch, b);
+    b = sq.b;
+    qs = sq.qs;
+    ks = sq.ks;
+    Sq = sq.Sq;
+    Sk = sq.Sk;
   }
   const int key0 = nb * BN;
   if (key0 >= Sk) return;

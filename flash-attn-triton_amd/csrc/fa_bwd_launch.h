@@ -6,6 +6,8 @@
 #include "fa_bwd_kernel.h"
 #include "fa_bwd_split.h"
 
+#include <algorithm>
+
 namespace fa {
 
 // dQ: 4 waves x 32 query rows, 64-key tiles (32 from D = 128, where Q, dO and
@@ -36,19 +38,22 @@ hipError_t launch_dkdv(BwdParams p, hipStream_t st) {
   if (total > 0x7fffffff) return hipErrorInvalidConfiguration;
   if (total <= 0) return hipSuccess;
   p.total_blocks = (int)total;
+  p.span = l2_span(p.seqlen_q, D, p.group, 1, VARLEN ? 1 : 2);
   hipLaunchKernelGGL(kern, dim3((unsigned)total), dim3(Tile::NT), (unsigned)lds, st, p);
   return hipGetLastError();
 }
 
-// dK/dV for D <= 128: a P-wave and a dS-wave per group of 32 keys, 128 keys
-// per workgroup, 4 LDS stages.
-template <class T, int D, bool GEN, bool VARLEN, bool BIAS>
-hipError_t launch_dkdv_split(BwdParams p, hipStream_t st) {
-  // 32 query rows per tile from D = 128, and for the generic D = 64 kernels
-  // (whose elementwise step needs the registers); 64 below.
-  constexpr int BM = D >= 128 || (GEN && D >= 64) ? 32 : 64;
-  using Tile = BwdDkvSplitTile<T, D, BM, 4>;
-  auto kern = bwd_dkdv_split_kernel<T, D, BM, 4, GEN, VARLEN, BIAS>;
+// dK/dV for D <= 128 (fa_bwd_split.h): a P-wave and a dS-wave per group of 32
+// keys, 128 keys per workgroup and 4 LDS stages; with ST = 2 two pairs of waves
+// per group, 64 keys and 3 stages.
+template <class T, int D, int ST, bool GEN, bool VARLEN, bool BIAS>
+hipError_t launch_dkdv_split_st(BwdParams p, hipStream_t st) {
+  // 32 query rows per pair and tile from D = 128, and for the generic D = 64
+  // kernels (whose elementwise step needs the registers); 64 below.
+  constexpr int BM = ST == 2 ? 64 : D >= 128 || (GEN && D >= 64) ? 32 : 64;
+  constexpr int NS = ST == 2 ? 3 : 4;
+  using Tile = BwdDkvSplitTile<T, D, BM, NS, ST>;
+  auto kern = bwd_dkdv_split_kernel<T, D, BM, NS, ST, GEN, VARLEN, BIAS>;
   constexpr int kMaxLds = 160 * 1024;
   static std::atomic<uint64_t> lds_devices{0};
   hipError_t e = set_lds_limit(lds_devices, kern, kMaxLds);
@@ -60,8 +65,28 @@ hipError_t launch_dkdv_split(BwdParams p, hipStream_t st) {
   if (total > 0x7fffffff) return hipErrorInvalidConfiguration;
   if (total <= 0) return hipSuccess;
   p.total_blocks = (int)total;
+  p.span = l2_span(p.seqlen_q, D, p.group, 1, VARLEN ? 1 : 2);
   hipLaunchKernelGGL(kern, dim3((unsigned)total), dim3(Tile::NT), (unsigned)lds, st, p);
   return hipGetLastError();
+}
+
+// ST = 2 where few workgroups have keys: up to 300 of 128 keys (causal, whose
+// workgroups average half the longest chain) or 150.  Measured on one MI355X,
+// whole backward, ST = 1 -> 2, B / S / Hq / Hk / D, workgroups: causal 1 / 4096 /
+// 8 / 2 / 128 (64) 504 -> 348 us, 2 / 2048 / 32 / 8 / 128 (256) 323 -> 273, 2 /
+// 2048 / 8 / 8 / 64 (256) 78 -> 68, 5 / 2048 / 4 / 4 / 128 (320) 152 -> 156, 3 /
+// 2048 / 8 / 8 / 128 (384) 129 -> 135; not causal 1 / 4096 / 4 / 4 / 128 (128) 207
+// -> 175, 2 / 1536 / 8 / 8 / 128 (192) 89 -> 101.  (The generic kernels' second
+// form would not pay for its instantiations.)
+template <class T, int D, bool GEN, bool VARLEN, bool BIAS>
+hipError_t launch_dkdv_split(const BwdParams& p, hipStream_t st) {
+  if constexpr (!GEN && (D == 64 || D == 128)) {
+    int64_t wgs = (int64_t)((p.seqlen_k + 127) / 128) * p.heads_k * p.batch;
+    if (VARLEN && p.total_k > 0)   // on average half a workgroup more than its keys fill per sequence
+      wgs = std::min(wgs, (p.total_k / 128 + (p.batch + 1) / 2) * p.heads_k);
+    if (wgs <= (p.causal ? 300 : 150)) return launch_dkdv_split_st<T, D, 2, GEN, VARLEN, BIAS>(p, st);
+  }
+  return launch_dkdv_split_st<T, D, 1, GEN, VARLEN, BIAS>(p, st);
 }
 
 template <class T, int D, bool GEN, bool VARLEN, bool BIAS>
@@ -78,6 +103,9 @@ hipError_t launch_bwd_v(BwdParams p, hipStream_t st) {
     if (total > 0x7fffffff) return hipErrorInvalidConfiguration;
     if (total > 0) {
       p.total_blocks = (int)total;
+      // (query heads of one K/V head share its tiles; the varlen order counts
+      // K/V heads)
+      p.span = l2_span(p.seqlen_k, D, 1, VARLEN ? 1 : p.group, VARLEN ? 1 : 2);
       hipLaunchKernelGGL(kern, dim3((unsigned)total), dim3(Tile::NT), Tile::LDS_BYTES, st, p);
       e = hipGetLastError();
       if (e != hipSuccess) return e;

@@ -30,39 +30,49 @@
 
 namespace fa {
 
-// Q and dO tiles of BM rows in NS LDS stages (DMA issued two tiles ahead, so
+// Q and dO tiles of BM rows in NS LDS stages (DMA issued NS - 2 tiles ahead, so
 // the stage of tile t - 1, which the dS-waves read while the P-waves work on
 // tile t, is not refilled before both are done with it), followed by two P
-// exchange buffers (tile parity) of 32 keys x BM rows in fp32 per key group.
-template <class T, int D, int BM, int NS>
+// exchange buffers (tile parity) of 32 keys x the rows of a pair in fp32 per
+// wave pair.
+//
+// ST = 2: two pairs of waves per key group, each with one half of every tile's
+// rows and accumulators of its own, which are summed through LDS at the end;
+// the workgroup then has two key groups instead of four.  A workgroup walks the
+// query tiles of every head of its GQA group, so with few workgroups its chain
+// of tiles is the kernel's time; this form makes the chain half as long and the
+// workgroups twice as many, for twice the tile loads per key.
+template <class T, int D, int BM, int NS, int ST>
 struct BwdDkvSplitTile {
-  static constexpr int KG = 4;                   // key groups of 32 keys
-  static constexpr int NW = 2 * KG;              // a P-wave and a dS-wave per group
+  static constexpr int KG = 4 / ST;              // key groups of 32 keys
+  static constexpr int NW = 2 * KG * ST;         // a P-wave and a dS-wave per pair
   static constexpr int BN = 32 * KG;
+  static constexpr int WM = BM / ST;             // rows of a pair per tile
   static constexpr int NT = 64 * NW;
   static constexpr int TILEB = BM * D * 2;       // bytes of one Q or dO stage
   static constexpr int IPS = TILEB / 1024;       // 1-KiB DMA instructions per Q (or dO) stage
   static constexpr int IPW = 2 * IPS / NW;       // per wave: waves [0, NW/2) load Q, the rest dO
   static constexpr int LPS = IPW + 1;            // DMA instructions per wave per stage (+ LSE or delta)
   static constexpr int FB = 256;                 // bytes of one LSE / delta stage
-  static constexpr int PB = 32 * BM * 4;         // fp32 P of one key group and tile
+  static constexpr int PB = 32 * WM * 4;         // fp32 P of one pair and tile
   static constexpr int STAGES_B = NS * (2 * TILEB + 2 * FB);
-  static constexpr int LDS_BYTES = STAGES_B + 2 * KG * PB;   // + 4 B per head of the group (ALiBi)
+  static constexpr int LDS_BYTES = STAGES_B + 2 * KG * ST * PB;   // + 4 B per head of the group (ALiBi)
   static_assert(IPW * NW == 2 * IPS && IPW > 0, "Q and dO tiles must split evenly over the waves");
-  static_assert(BM <= 64 && BM % 32 == 0, "one DMA lane per row for LSE / delta");
+  static_assert(BM <= 64 && WM % 32 == 0, "one DMA lane per row for LSE / delta");
+  static_assert(ST == 1 || NW / 2 * 128 * D <= LDS_BYTES, "the second pairs' sums must fit");
   static_assert(NW * 32 * (2 * D + 16) <= LDS_BYTES, "output staging must fit");
 };
 
-template <class T, int D, int BM, int NS, bool GENERIC, bool VARLEN, bool BIAS = false>
+template <class T, int D, int BM, int NS, int ST, bool GENERIC, bool VARLEN, bool BIAS = false>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void bwd_dkdv_split_kernel(const BwdParams p) {
   static_assert(!BIAS || (GENERIC && !VARLEN), "attn_bias: generic dense kernels only");
-  static_assert(NS == 4, "the loops are unrolled for four stages");
-  using Tile = BwdDkvSplitTile<T, D, BM, NS>;
+  using Tile = BwdDkvSplitTile<T, D, BM, NS, ST>;
   constexpr int KG = Tile::KG, BN = Tile::BN, NW = Tile::NW, TILEB = Tile::TILEB;
   constexpr int IPW = Tile::IPW, LPS = Tile::LPS, FB = Tile::FB, PB = Tile::PB;
-  constexpr int NKC = D / 16, NDB = D / 32, NRB = BM / 32, NCC = BM / 16;
-  constexpr int PD = 2;                          // DMA distance in tiles
+  constexpr int WM = Tile::WM;
+  constexpr int NKC = D / 16, NDB = D / 32, NRB = WM / 32, NCC = WM / 16;
+  constexpr int PD = NS - 2;                     // DMA distance in tiles
 
   extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
   uint8_t* const smem_b = reinterpret_cast<uint8_t*>(smem);
@@ -73,25 +83,29 @@ void bwd_dkdv_split_kernel(const BwdParams p) {
   const int lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int grp = w % KG;                        // key group
-  const bool dsw = w >= KG;                      // the dS-wave of the group
+  const bool dsw = w >= KG * ST;                 // the dS-wave of the pair (on its P-wave's SIMD)
+  const int pair = w % (KG * ST);
+  const int srow = ST == 1 ? 0 : pair / KG * WM; // first row of the pair's part of every tile
   const int c32 = lane & 31;
   const int g = lane >> 5;
 
   // ------------------------------------------------------------ work item
   int nb, id;
   if (!VARLEN ||
-      !work_item_kv_rr(blockIdx.x, p.total_blocks, p.n_blocks, 1, p.causal != 0, nb, id))
-    work_item(blockIdx.x, p.total_blocks, p.n_blocks, p.causal != 0, kBwdCausalSpan, nb, id);
+      !work_item_kv_rr(blockIdx.x, p.total_blocks, p.n_blocks, 1, p.causal != 0, p.span, nb, id))
+    work_item(blockIdx.x, p.total_blocks, p.n_blocks, p.causal != 0, p.span, nb, id);
   if (p.causal) nb = p.n_blocks - 1 - nb;
   const int kvh = id % p.heads_k;
-  const int b = id / p.heads_k;
+  int b = id / p.heads_k;
 
   int Sq = p.seqlen_q, Sk = p.seqlen_k, qs = 0, ks = 0;
-  if (p.cu_q != nullptr) {
-    qs = p.cu_q[b];
-    ks = p.cu_k[b];
-    Sq = p.cu_q[b + 1] - qs;
-    Sk = p.cu_k[b + 1] - ks;
+  if constexpr (VARLEN) {
+    const VarlenSeq sq = nth_longest(p.cu_q, p.cu_k, p.batch, b);
+    b = sq.b;
+    qs = sq.qs;
+    ks = sq.ks;
+    Sq = sq.Sq;
+    Sk = sq.Sk;
   }
   const int key0 = nb * BN;
   if (key0 >= Sk) return;
@@ -148,7 +162,7 @@ void bwd_dkdv_split_kernel(const BwdParams p) {
   if (wl >= 0) vis_hi = (int)min((int64_t)kj + wl, (int64_t)INT_MAX);
   const uint32_t vis_span = (uint32_t)vis_hi - (uint32_t)vis_lo;
   auto wave_masks = [&](int m0) {
-    const int p0 = m0 + qoff, p1 = m0 + BM - 1 + qoff;
+    const int p0 = m0 + qoff, p1 = m0 + WM - 1 + qoff;
     bool need = false;
     if (causal) need = need || p0 < wk1;
     if (wr >= 0) need = need || p0 + wr < wk1;
@@ -219,14 +233,14 @@ void bwd_dkdv_split_kernel(const BwdParams p) {
   for (int rb = 0; rb < NRB; ++rb)
 #pragma unroll
     for (int kc = 0; kc < NKC; ++kc)
-      rd_ofs[rb * NKC + kc] = 2u * (uint32_t)swz_off<D>(rb * 32 + c32, 2 * kc + g);
+      rd_ofs[rb * NKC + kc] = 2u * (uint32_t)swz_off<D>(srow + rb * 32 + c32, 2 * kc + g);
   {
     const int j = lane & 15;
 #pragma unroll
     for (int cc = 0; cc < NCC; ++cc)
 #pragma unroll
       for (int db = 0; db < NDB; ++db) {
-        const int r = 16 * cc + 4 * g + (j >> 2);
+        const int r = srow + 16 * cc + 4 * g + (j >> 2);
         const int d = db * 32 + 16 * (c32 >> 4) + 4 * (j & 3);
         tr_ofs[(cc * NDB + db) * 2] = 2u * (uint32_t)(swz_off<D>(r, d >> 3) + (d & 7));
         tr_ofs[(cc * NDB + db) * 2 + 1] = 2u * (uint32_t)(swz_off<D>(r + 8, d >> 3) + (d & 7));
@@ -282,7 +296,7 @@ void bwd_dkdv_split_kernel(const BwdParams p) {
     }
   };
   auto p_of = [&](int pslot) {   // this lane's slice of a P exchange buffer
-    return reinterpret_cast<float*>(pbuf + (pslot * KG + grp) * PB) + lane * 4;
+    return reinterpret_cast<float*>(pbuf + (pslot * KG * ST + pair) * PB) + lane * 4;
   };
 
   // P-wave, one tile in stage `stage`: S, P (written to the exchange buffer
@@ -290,9 +304,9 @@ void bwd_dkdv_split_kernel(const BwdParams p) {
   auto p_tile = [&](int stage, int pslot) __attribute__((always_inline)) {
     const uint8_t* Qb = smem_b + stage * TILEB;
     const uint8_t* Db = smem_b + (NS + stage) * TILEB;
-    const float* Ls = reinterpret_cast<const float*>(smem_b + 2 * NS * TILEB + stage * FB);
+    const float* Ls = reinterpret_cast<const float*>(smem_b + 2 * NS * TILEB + stage * FB) + srow;
     float* const Pw = p_of(pslot);
-    const int hq = kvh * p.group + mm_h, m0 = mm_m * BM;
+    const int hq = kvh * p.group + mm_h, m0 = mm_m * BM + srow;
     f32x16 sp[NRB];
     row_products(Qb, sp);
     // The transposed reads go ahead of the elementwise step, which hides
@@ -356,9 +370,9 @@ void bwd_dkdv_split_kernel(const BwdParams p) {
   // dS from the P in exchange buffer `pslot`, dK^T += Q^T dS.
   auto ds_tile = [&](const f32x16 (&dp)[NRB], int stage, int pslot) __attribute__((always_inline)) {
     const uint8_t* Qb = smem_b + stage * TILEB;
-    const float* Es = reinterpret_cast<const float*>(smem_b + 2 * NS * TILEB + (NS + stage) * FB);
+    const float* Es = reinterpret_cast<const float*>(smem_b + 2 * NS * TILEB + (NS + stage) * FB) + srow;
     const float* Pw = p_of(pslot);
-    const int hq = kvh * p.group + mm_h, m0 = mm_m * BM;
+    const int hq = kvh * p.group + mm_h, m0 = mm_m * BM + srow;
     u32x4 ta[NTA];
     if constexpr (!GENERIC) tr_operands(Qb, ta);
     u32x4 bop[NCC];
@@ -412,30 +426,40 @@ void bwd_dkdv_split_kernel(const BwdParams p) {
     __builtin_amdgcn_sched_barrier(0);
     issue((ts + PD) % NS);
   };
+  // round(t, t % NS, t % 2), unrolled so that stage and parity are constants.
   auto unrolled = [&](auto&& round) __attribute__((always_inline)) {
-    int t = 0;
-    for (; t + NS <= J + 1; t += NS) {
-      round(t, 0);
-      round(t + 1, 1);
-      round(t + 2, 2);
-      round(t + 3, 3);
+    if constexpr (NS == 4) {
+      int t = 0;
+      for (; t + NS <= J + 1; t += NS) {
+        round(t, 0, 0);
+        round(t + 1, 1, 1);
+        round(t + 2, 2, 0);
+        round(t + 3, 3, 1);
+      }
+      if (t < J + 1) round(t, 0, 0);
+      if (t + 1 < J + 1) round(t + 1, 1, 1);
+      if (t + 2 < J + 1) round(t + 2, 2, 0);
+    } else {
+      static_assert(NS == 3, "three or four stages");
+      for (int t = 0; t < J + 1; t += 2 * NS) {
+#pragma unroll
+        for (int u = 0; u < 2 * NS; ++u)
+          if (u == 0 || t + u < J + 1) round(t + u, u % NS, u & 1);
+      }
     }
-    if (t < J + 1) round(t, 0);
-    if (t + 1 < J + 1) round(t + 1, 1);
-    if (t + 2 < J + 1) round(t + 2, 2);
   };
   if (!dsw) {
-    unrolled([&](int t, int ts) __attribute__((always_inline)) {
+    unrolled([&](int t, int ts, int par) __attribute__((always_inline)) {
       top(ts);
-      if (t < J) p_tile(ts, ts & 1);
+      if (t < J) p_tile(ts, par);
     });
   } else {
     f32x16 dp[NRB];
 #pragma unroll
     for (int rb = 0; rb < NRB; ++rb) dp[rb] = f32x16{};
-    unrolled([&](int t, int ts) __attribute__((always_inline)) {
+    unrolled([&](int t, int ts, int par) __attribute__((always_inline)) {
       top(ts);
-      if (t >= 1) ds_tile(dp, (ts + NS - 1) % NS, (ts + 1) & 1);
+      if (t >= 1) ds_tile(dp, (ts + NS - 1) % NS, par ^ 1);
       if (t < J) row_products(smem_b + (NS + ts) * TILEB, dp);
     });
   }
@@ -443,6 +467,28 @@ void bwd_dkdv_split_kernel(const BwdParams p) {
 
   // ------------------------------------------------------------ dK = scale * dK^T, dV
   __syncthreads();
+  if constexpr (ST == 2) {
+    // The second pair's sums join the first's (fp32, 16 bytes per lane).
+    float* const xs = reinterpret_cast<float*>(smem_b) + ((w / (KG * ST)) * KG + grp) * 32 * D + lane * 4;
+    if (srow != 0) {
+#pragma unroll
+      for (int i = 0; i < NDB * 4; ++i)
+        *reinterpret_cast<f32x4*>(xs + i * 256) =
+            f32x4{acc[i >> 2][4 * (i & 3)], acc[i >> 2][4 * (i & 3) + 1], acc[i >> 2][4 * (i & 3) + 2],
+                  acc[i >> 2][4 * (i & 3) + 3]};
+    }
+    __syncthreads();
+    if (srow == 0) {
+#pragma unroll
+      for (int i = 0; i < NDB * 4; ++i) {
+        const f32x4 x = *reinterpret_cast<const f32x4*>(xs + i * 256);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[i >> 2][4 * (i & 3) + e] += x[e];
+      }
+    }
+    __syncthreads();
+    if (srow != 0) return;
+  }
   uint8_t* const st = smem_b + w * 32 * (2 * D + 16);
   const int rows_ok = Sk - wk0;
   if (dsw)

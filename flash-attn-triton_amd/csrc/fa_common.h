@@ -11,6 +11,8 @@
 
 #include "fa_fastdiv.h"
 
+#include <limits.h>
+
 #include <atomic>
 
 namespace fa {
@@ -168,43 +170,94 @@ __device__ inline void work_item(int L, int total, int n_mblocks, bool heavy_fir
 
 // Work item of a varlen launch, whose groups differ in work (their
 // sequences' lengths): contiguous group ranges per XCD would load the XCDs
-// unevenly (1.56x the mean on the busiest XCD at 32 random lengths).  Here
-// XCD x owns the K/V heads c = grp / group with c % 8 == x, so the sequences
-// spread over all XCDs while the query heads of one K/V head share its tiles
-// in one L2, and runs them one K/V head at a time (row blocks of the head's
-// query heads interleaved, the last first when heavy_first).  The last
-// n_kv % 8 K/V heads, if any, follow with their items spread over all XCDs.
+// unevenly (1.56x the mean on the busiest XCD at 32 random lengths).  Here the
+// K/V heads c = grp / group are dealt round-robin over the XCDs, back and forth
+// (with the sequences taken longest first, nth_longest, that evens out the
+// XCDs), so the query heads of one K/V head share its tiles in one L2, and an
+// XCD runs them `span` K/V heads at a time (row blocks of the heads' query
+// heads interleaved, the last first when heavy_first).  The last n_kv % 8 K/V
+// heads, if any, follow with their items spread over all XCDs.
 // Returns false (no item assigned) unless total = n_kv * group * n_mblocks.
 __device__ inline bool work_item_kv_rr(int L, int total, int n_mblocks, int group,
-                                       bool heavy_first, int& mb, int& grp) {
+                                       bool heavy_first, int span, int& mb, int& grp) {
   constexpr int kXcds = 8;
   const int per_kv = group * n_mblocks;   // items per K/V head
   if (per_kv <= 0 || total % per_kv != 0) return false;
-  const int main_items = total / per_kv / kXcds * kXcds * per_kv;
-  int c, r;
-  if (L < main_items) {
-    const int k = L / kXcds;
-    c = (k / per_kv) * kXcds + L % kXcds;
-    r = k % per_kv;
-  } else {
-    c = L / per_kv;   // main_items is a multiple of per_kv
-    r = L % per_kv;
-  }
-  mb = r / group;
+  const int heads = total / per_kv / kXcds;   // whole rounds of K/V heads over the XCDs
+  const bool main = L < heads * kXcds * per_kv;
+  const int k = main ? L / kXcds : L - heads * kXcds * per_kv;
+  const int k0 = k / (span * per_kv) * span;   // this span's first round (tail: first head)
+  const int cw = min(span, (main ? heads : total / per_kv - heads * kXcds) - k0);
+  int r = k - k0 * per_kv;
+  mb = r / (group * cw);
+  r -= mb * group * cw;
   if (heavy_first) mb = n_mblocks - 1 - mb;
+  const int round = k0 + r / group, x = L % kXcds;
+  const int c = main ? round * kXcds + (round & 1 ? kXcds - 1 - x : x) : heads * kXcds + round;
   grp = c * group + r % group;
   return true;
+}
+
+// The r-th longest sequence (by queries; r counted within its block of 64
+// consecutive ones) of the n that cu_q and cu_k describe, with its offsets and
+// lengths; every lane of the wave takes part.  A varlen launch hands its
+// sequences out in this order, so that the long ones do not start last and the
+// XCDs get even shares.  It takes the place of the scalar reads of the four
+// offsets (one trip to memory either way) and adds three instructions per
+// sequence.  Measured on one MI355X, causal, forward / backward, before and
+// after (with the spans below): 8 sequences of 150 to 1999 tokens, Hq16 Hk4
+// D128 bf16, 97.5 / 351 -> 79.6 / 292 us; 20 of 300 and 2000, H16 D64 fp16, 75.6
+// / 294 -> 69.9 / 262 us; 24 of 128 to 2428, H16 D128 bf16, 307 / 983 -> 306 /
+// 995 us.
+struct VarlenSeq {
+  int b, qs, Sq, ks, Sk;
+};
+__device__ inline VarlenSeq nth_longest(const int* cu_q, const int* cu_k, int n, int r) {
+  const int base = r & ~63, m = min(64, n - base), l = threadIdx.x & 63;
+  int q0 = 0, q1 = 0, k0 = 0, k1 = 0;
+  if (l < m) {
+    q0 = cu_q[base + l];
+    q1 = cu_q[base + l + 1];
+    k0 = cu_k[base + l];
+    k1 = cu_k[base + l + 1];
+  }
+  // Unique keys: the length (clamped), then the earlier sequence.
+  const uint32_t key = ((uint32_t)min(q1 - q0, (1 << 25) - 2) << 6) + 64u + (uint32_t)(63 - l);
+  int rank = 0;
+  for (int j0 = 0; j0 < m; j0 += 8) {   // (lanes past m hold keys below every sequence's)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) rank += (uint32_t)__builtin_amdgcn_readlane(key, j0 + j) > key ? 1 : 0;
+  }
+  const uint64_t hit = __builtin_amdgcn_ballot_w64(l < m && rank == (r & 63));
+  const int i = hit != 0 ? (int)__builtin_ctzll(hit) : 0;
+  VarlenSeq s;
+  s.b = base + i;
+  s.qs = __builtin_amdgcn_readlane(q0, i);
+  s.Sq = __builtin_amdgcn_readlane(q1, i) - s.qs;
+  s.ks = __builtin_amdgcn_readlane(k0, i);
+  s.Sk = __builtin_amdgcn_readlane(k1, i) - s.ks;
+  return s;
 }
 
 // work_item span of the causal launches of the ping-pong forward and INT8
 // kernels (and of the fp32 backward): 4 groups measured best on MI355X at
 // B=4 H=32 S=4096 (1: 5-7% slower, all groups of an XCD: 1-3% slower).
 constexpr int kCausalSpan = 4;
-// The 16-bit backward kernels' span: each group streams 2 MiB of K / V (dQ)
-// or Q / dO (dK/dV) per XCD at that shape, so four groups at a time
-// overflowed the 4 MiB L2 (causal dQ + dK/dV read 1882 MB for 672 MB of
-// inputs); two read 1333 MB for 0.9% more time, one 1367 MB for 5.4%.
-constexpr int kBwdCausalSpan = 2;
+// Spans that keep what an XCD streams at a time within its 4 MiB L2: as many
+// groups as stream 4 MiB of K / V (forward, dQ) or Q / dO (dK/dV), `rows` long,
+// `heads_streamed` heads per group (or one for `heads_sharing` groups), and at
+// least `least`.  The 16-bit backward kernels at B=4 H=32 S=4096 D=128 (2 MiB
+// per group): four groups at a time read 1882 MB for 672 MB of inputs; two (the
+// least of the dense launches) read 1333 MB for 0.9% more time, one 1367 MB for
+// 5.4%.  Shorter sequences take more: at B=8 H=16 S=1024
+// D=64 causal the backward went from 139 to 115 us, at B=3 H=8 S=2048 D=128 from
+// 154 to 129 us.
+inline int l2_span(int64_t rows, int64_t head_dim, int64_t heads_streamed, int64_t heads_sharing,
+                   int least) {
+  const int64_t bytes = 4 * (rows > 0 ? rows : 1) * head_dim * heads_streamed;   // both tensors
+  const int64_t n = (int64_t(4) << 20) * heads_sharing / bytes;
+  return (int)(n < least ? least : n > 4096 ? 4096 : n);
+}
 
 __device__ inline u32x4 load16(const void* p) { return *reinterpret_cast<const u32x4*>(p); }
 __device__ inline void store16(void* p, u32x4 v) { *reinterpret_cast<u32x4*>(p) = v; }

@@ -105,7 +105,8 @@ void prefill_d64_kernel(const FwdParams p) {
   } else {
     int id;
     if (!VARLEN ||
-        !work_item_kv_rr(blockIdx.x, p.total_blocks, p.n_mblocks, p.group, p.heavy_first != 0, mb, id))
+        !work_item_kv_rr(blockIdx.x, p.total_blocks, p.n_mblocks, p.group, p.heavy_first != 0, p.span, mb,
+                         id))
       work_item(blockIdx.x, p.total_blocks, p.n_mblocks, p.heavy_first != 0, p.span, mb, id);
     hh = id % p.heads_q;
     b = id / p.heads_q;
@@ -116,12 +117,13 @@ void prefill_d64_kernel(const FwdParams p) {
   int64_t q_base, o_base, lse_base, k_base = 0, v_base = 0;
   typedef const __attribute__((address_space(4))) int* table_ptr;
   table_ptr bt_row = nullptr;
-  if constexpr (PAGED) bt_row = (table_ptr)(p.block_table + (int64_t)b * p.bt_stride);
   if constexpr (VARLEN) {
     if (guard_failed(p)) return;
-    const int qs = p.cu_q[b], ks = p.cu_k[b];
-    Sq = p.cu_q[b + 1] - qs;
-    Sk = p.cu_k[b + 1] - ks;
+    const VarlenSeq sq = nth_longest(p.cu_q, p.cu_k, p.batch, b);
+    const int qs = sq.qs, ks = sq.ks;
+    b = sq.b;
+    Sq = sq.Sq;
+    Sk = sq.Sk;
     if (p.seqused_q != nullptr) Sq = max(0, min(Sq, p.seqused_q[b]));
     if (p.seqused_k != nullptr) Sk = max(0, min(Sk, p.seqused_k[b]));
     const int os = p.cu_o != nullptr ? p.cu_o[b] : qs;
@@ -153,6 +155,7 @@ void prefill_d64_kernel(const FwdParams p) {
       v_base = (int64_t)b * p.v_sb;
     }
   }
+  if constexpr (PAGED) bt_row = (table_ptr)(p.block_table + (int64_t)b * p.bt_stride);
   q_base += (int64_t)hh * p.q_sh;
   o_base += (int64_t)hh * p.o_sh;
   lse_base += (int64_t)hh * p.lse_sh;

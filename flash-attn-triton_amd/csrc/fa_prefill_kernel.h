@@ -122,19 +122,21 @@ void prefill_kernel(const FwdParams p) {
   // the varlen configuration.
   int mb, id;
   if (p.cu_q == nullptr ||
-      !work_item_kv_rr(blockIdx.x, p.total_blocks, p.n_mblocks, p.group, p.heavy_first != 0, mb, id))
+      !work_item_kv_rr(blockIdx.x, p.total_blocks, p.n_mblocks, p.group, p.heavy_first != 0, 1, mb, id))
     work_item(blockIdx.x, p.total_blocks, p.n_mblocks, p.heavy_first != 0, 1, mb, id);
+  if (guard_failed(p)) return;
   const int hh = id % p.heads_q;
-  const int b = id / p.heads_q;
+  int b = id / p.heads_q;
   const int kvh = hh / p.group;
 
   int Sq, Sk;
   int64_t q_base, o_base, lse_base, k_base, v_base;
-  if (guard_failed(p)) return;
   if (p.cu_q != nullptr) {
-    const int qs = p.cu_q[b], ks = p.cu_k[b];
-    Sq = p.cu_q[b + 1] - qs;
-    Sk = p.cu_k[b + 1] - ks;
+    const VarlenSeq sq = nth_longest(p.cu_q, p.cu_k, p.batch, b);
+    const int qs = sq.qs, ks = sq.ks;
+    b = sq.b;
+    Sq = sq.Sq;
+    Sk = sq.Sk;
     if (p.seqused_q != nullptr) Sq = max(0, min(Sq, p.seqused_q[b]));
     if (p.seqused_k != nullptr) Sk = max(0, min(Sk, p.seqused_k[b]));
     const int os = p.cu_o != nullptr ? p.cu_o[b] : qs;

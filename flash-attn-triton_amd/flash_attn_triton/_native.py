@@ -59,6 +59,9 @@ _SIGNATURES = {
                       _i64p, _f32, _u64, _vp]),
     "fa_bwd_varlen": (_int, [_vp] * 12 + [_i64] * 6 + [_i64p] * 9 +
                       [_int, _f32, _int, _i64, _i64, _f32, _vp, _i64, _f32, _u64, _vp]),
+    "fa_bwd_varlen_sized": (_int, [_vp] * 12 + [_i64] * 6 + [_i64p] * 9 +
+                            [_int, _f32, _int, _i64, _i64, _f32, _vp, _i64, _f32, _u64, _i64,
+                             _vp]),
     "fa_fwd_kvcache_plan": (_int, [_i64, _i64, _i64, _i64, _i64, _i64, _i64, _i32p, _i64p]),
     "fa_fwd_kvcache": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _vp,
                               _i64, _i64, _i64, _i64, _i64, _i64, _i64p, _i64p, _i64p, _i64p,
@@ -205,13 +208,13 @@ def bwd_varlen(q, k, v, out, dout, lse, dq, dk, dv, delta, cu_q, cu_k, max_seqle
     Hq, D = q.shape[1], q.shape[2]
     Hk = k.shape[1]
     st = [_strides(t.stride()[:2]) for t in (q, k, v, out, dout, dq, dk, dv)]
-    status = lib.fa_bwd_varlen(
+    status = lib.fa_bwd_varlen_sized(
         _ptr(q), _ptr(k), _ptr(v), _ptr(out), _ptr(dout), _ptr(lse), _ptr(dq), _ptr(dk),
         _ptr(dv), _ptr(delta), _ptr(cu_q), _ptr(cu_k), cu_q.numel() - 1, int(max_seqlen_q),
         int(max_seqlen_k), Hq, Hk, D, *st, _strides(lse.stride()), dtype_code(q.dtype),
         float(softmax_scale), int(bool(causal)), int(window_left), int(window_right),
         float(softcap), _ptr(alibi), 0 if alibi is None else int(alibi.stride(0)),
-        float(dropout_p), int(dropout_seed), _stream(q.device))
+        float(dropout_p), int(dropout_seed), k.shape[0], _stream(q.device))
     _check(status, "fa_bwd_varlen")
 
 

@@ -201,6 +201,21 @@ int fa_bwd_varlen(const void* q, const void* k, const void* v, const void* out,
                   const float* alibi_slopes, int64_t alibi_batch_stride, float dropout_p,
                   uint64_t dropout_seed, fa_stream_t stream);
 
+/* fa_bwd_varlen with the number of packed keys (cu_seqlens_k[batch], which the
+ * caller knows from its tensors; 0: unknown): the launch chooses its tiles by
+ * how many of them hold keys. */
+int fa_bwd_varlen_sized(const void* q, const void* k, const void* v, const void* out,
+                  const void* dout, const float* lse, void* dq, void* dk, void* dv, float* delta,
+                  const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, int64_t batch,
+                  int64_t max_seqlen_q, int64_t max_seqlen_k, int64_t heads_q, int64_t heads_k,
+                  int64_t head_dim, const int64_t* q_stride, const int64_t* k_stride,
+                  const int64_t* v_stride, const int64_t* o_stride, const int64_t* do_stride,
+                  const int64_t* dq_stride, const int64_t* dk_stride, const int64_t* dv_stride,
+                  const int64_t* lse_stride, int dtype, float softmax_scale, int causal,
+                  int64_t window_left, int64_t window_right, float softcap,
+                  const float* alibi_slopes, int64_t alibi_batch_stride, float dropout_p,
+                  uint64_t dropout_seed, int64_t total_k, fa_stream_t stream);
+
 /* Split-KV plan for fa_fwd_kvcache: the number of key splits the launch will
  * use and the workspace bytes it needs (0 when num_splits == 1).
  * max_keys bounds every sequence's visible key count (e.g. the cache
