@@ -46,6 +46,7 @@ from .triton_kernel.attention_kernel import (
     dense_attention,
     dense_forward,
     new_dropout_seed,
+    unpack,
     varlen_attention,
     varlen_forward,
 )
@@ -183,6 +184,13 @@ def flash_attn_func(q, k, v, dropout_p=0.0, softmax_scale=None, causal=False,
     Return:
         out: (batch_size, seqlen, nheads, headdim).
     """
+    return _dense(q, k, v, dropout_p, softmax_scale, causal, window_size, softcap, alibi_slopes,
+                  deterministic, return_attn_probs, use_native_gqa, attn_bias)
+
+
+def _dense(q, k, v, dropout_p, softmax_scale, causal, window_size, softcap, alibi_slopes,
+           deterministic, return_attn_probs, use_native_gqa, attn_bias, packed=0):
+    """``flash_attn_func``; the last ``packed`` of q, k, v come from ``unpack``."""
     if q.dtype not in (torch.float16, torch.bfloat16, torch.float32):
         raise ValueError("This implementation supports FP16, BF16 and FP32 tensors")
     if softcap < 0.0:
@@ -224,12 +232,8 @@ def flash_attn_func(q, k, v, dropout_p=0.0, softmax_scale=None, causal=False,
                                      softcap, alibi_slopes, attn_bias)[0]
 
     if seq_len_q != seq_len_k:
-        return flash_attn_func_cross(
-            q, k, v, dropout_p=dropout_p, softmax_scale=softmax_scale,
-            causal=causal, use_native_gqa=use_native_gqa, softcap=softcap,
-            alibi_slopes=alibi_slopes, window_size=window_size,
-            deterministic=deterministic,
-        )
+        return _cross(q, k, v, dropout_p, softmax_scale, causal, softcap, alibi_slopes, window_size,
+                      False, None, 0, packed)
     # Equal-length path: unsupported head dims surface as AssertionError, as in
     # the reference's _launch_dense_forward (attention_kernel.py:1063-1064).
     assert head_dim in {16, 32, 64, 128, 256}
@@ -239,7 +243,8 @@ def flash_attn_func(q, k, v, dropout_p=0.0, softmax_scale=None, causal=False,
                            window_left=window_size[0], window_right=window_size[1],
                            softcap=softcap, alibi=alibi_slopes if use_alibi else None,
                            dropout_p=dropout_p,
-                           dropout_seed=new_dropout_seed() if dropout_p > 0.0 else 0)
+                           dropout_seed=new_dropout_seed() if dropout_p > 0.0 else 0,
+                           packed=packed)
 
 
 def flash_attn_func_cross(q, k, v, dropout_p=0.0, softmax_scale=None, causal=False,
@@ -251,6 +256,13 @@ def flash_attn_func_cross(q, k, v, dropout_p=0.0, softmax_scale=None, causal=Fal
     Query row ``i`` sits at position ``i + _causal_offset`` (0: upper-left,
     the SDPA convention for rectangular masks).
     """
+    return _cross(q, k, v, dropout_p, softmax_scale, causal, softcap, alibi_slopes, window_size,
+                  return_attn_probs, attn_bias, _causal_offset)
+
+
+def _cross(q, k, v, dropout_p, softmax_scale, causal, softcap, alibi_slopes, window_size,
+           return_attn_probs, attn_bias, _causal_offset, packed=0):
+    """``flash_attn_func_cross``; the last ``packed`` of q, k, v come from ``unpack``."""
     if (q.dtype not in (torch.float16, torch.bfloat16, torch.float32) or k.dtype != q.dtype
             or v.dtype != q.dtype):
         raise ValueError("flash_attn_func_cross supports matching FP16, BF16 or FP32 tensors")
@@ -293,7 +305,8 @@ def flash_attn_func_cross(q, k, v, dropout_p=0.0, softmax_scale=None, causal=Fal
                            q_pos_offset=_causal_offset, window_left=window_size[0],
                            window_right=window_size[1], softcap=softcap,
                            alibi=alibi_slopes if use_alibi else None, dropout_p=dropout_p,
-                           dropout_seed=new_dropout_seed() if dropout_p > 0.0 else 0)
+                           dropout_seed=new_dropout_seed() if dropout_p > 0.0 else 0,
+                           packed=packed)
 
 
 def flash_attn_qkvpacked_func(qkv, dropout_p=0.0, softmax_scale=None, causal=False,
@@ -302,14 +315,15 @@ def flash_attn_qkvpacked_func(qkv, dropout_p=0.0, softmax_scale=None, causal=Fal
                               use_native_gqa=False, attn_bias=None):
     """Packed QKV (reference :337-371). qkv: (batch_size, seqlen, 3, nheads, headdim).
 
-    The three strided slices are read in place (token stride 3*H*D); the
-    reference copies each slice to a contiguous tensor first.
+    The three strided slices are read in place (token stride 3*H*D), and the
+    backward writes the packed gradient in place; the reference copies each
+    slice to a contiguous tensor first.  (Stacking three gradients took 36 us of
+    a 175 us forward + backward at B=8 S=1024 H=16 D=64 on MI355X.)
     """
     qkv = qkv.contiguous() if not qkv.is_contiguous() else qkv
-    q, k, v = qkv.unbind(dim=2)
-    return flash_attn_func(q, k, v, dropout_p, softmax_scale, causal, window_size, softcap,
-                           alibi_slopes, deterministic, return_attn_probs, use_native_gqa,
-                           attn_bias)
+    q, k, v = unpack(qkv, 2)
+    return _dense(q, k, v, dropout_p, softmax_scale, causal, window_size, softcap, alibi_slopes,
+                  deterministic, return_attn_probs, use_native_gqa, attn_bias, packed=3)
 
 
 def flash_attn_kvpacked_func(q, kv, dropout_p=0.0, softmax_scale=None, causal=False,
@@ -318,10 +332,9 @@ def flash_attn_kvpacked_func(q, kv, dropout_p=0.0, softmax_scale=None, causal=Fa
                              use_native_gqa=False, attn_bias=None):
     """Packed KV (reference :374-406). kv: (batch_size, seqlen_k, 2, nheads_k, headdim)."""
     kv = kv.contiguous() if not kv.is_contiguous() else kv
-    k, v = kv.unbind(dim=2)
-    return flash_attn_func(q, k, v, dropout_p, softmax_scale, causal, window_size, softcap,
-                           alibi_slopes, deterministic, return_attn_probs, use_native_gqa,
-                           attn_bias)
+    k, v = unpack(kv, 2)
+    return _dense(q, k, v, dropout_p, softmax_scale, causal, window_size, softcap, alibi_slopes,
+                  deterministic, return_attn_probs, use_native_gqa, attn_bias, packed=2)
 
 
 def _outlasts_the_host(q, k_cache, block_table) -> bool:
@@ -665,6 +678,15 @@ def flash_attn_varlen_func(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q,
     reference's compaction does (:551-581).  The kernels read the block
     table and the used counts directly: nothing is gathered or copied.
     """
+    return _varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, dropout_p,
+                   softmax_scale, causal, window_size, softcap, alibi_slopes, return_attn_probs,
+                   block_table, seqused_q, seqused_k)
+
+
+def _varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, dropout_p=0.0,
+            softmax_scale=None, causal=False, window_size=(-1, -1), softcap=0.0, alibi_slopes=None,
+            return_attn_probs=False, block_table=None, seqused_q=None, seqused_k=None, packed=0):
+    """``flash_attn_varlen_func``; the last ``packed`` of q, k, v come from ``unpack``."""
     batch_size = cu_seqlens_q.numel() - 1
     chk = Deferred()
     paged = block_table is not None
@@ -795,7 +817,10 @@ def flash_attn_varlen_func(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q,
         chk.fail(exc)
     # Any nonzero slope?  The fp32 bit patterns' range (one array of the
     # range-check launch): all slopes +0.0 iff min and max are both 0.
-    alibi_bits = chk.value_range(alibi.view(torch.int32)) if alibi is not None else None
+    # With softcap the kernel is the same either way (and zero slopes change no
+    # bit of its result), so the question is not asked.
+    ask_alibi = alibi is not None and not softcap > 0.0
+    alibi_bits = chk.value_range(alibi.view(torch.int32)) if ask_alibi else None
     if return_attn_probs:
         chk.flush()
         if paged or seqused_q is not None or seqused_k is not None:
@@ -805,7 +830,7 @@ def flash_attn_varlen_func(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q,
                                             max_seqlen_k, dropout_p, softmax_scale, causal,
                                             window_size, softcap, alibi)
     plain = not (paged or seqused_q is not None or seqused_k is not None)
-    if plain and alibi is None and chk.ranges_only():
+    if plain and not ask_alibi and chk.ranges_only():
         # Nothing below depends on a checked value: the launch goes out first,
         # guarded by the checks' device flags, and the host waits for the checks
         # (the one synchronization of this call) while it runs.
@@ -815,11 +840,12 @@ def flash_attn_varlen_func(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q,
         chk.flush(lambda guard: result.append(varlen_attention(
             q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, softmax_scale=scale,
             causal=causal, window_left=window_size[0], window_right=window_size[1],
-            softcap=softcap, dropout_p=dropout_p, dropout_seed=seed, guard=guard)), guarded=True)
+            softcap=softcap, alibi=alibi, dropout_p=dropout_p, dropout_seed=seed, guard=guard,
+            packed=packed, covered=True)), guarded=True)
         return result[0]
     values = chk.flush()   # the one host synchronization of this call
     seed = new_dropout_seed() if dropout_p > 0.0 else 0
-    use_alibi = alibi is not None and values[alibi_bits] != (0, 0)
+    use_alibi = alibi is not None and (not ask_alibi or values[alibi_bits] != (0, 0))
     if softmax_scale is None:
         softmax_scale = 1.0 / math.sqrt(q.shape[-1])
     cu_out = None
@@ -852,26 +878,35 @@ def flash_attn_varlen_func(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q,
                             softmax_scale=softmax_scale, causal=causal,
                             window_left=window_size[0], window_right=window_size[1],
                             softcap=softcap, alibi=alibi if use_alibi else None,
-                            dropout_p=dropout_p, dropout_seed=seed)
+                            dropout_p=dropout_p, dropout_seed=seed, packed=packed, covered=True)
+
+
+def _varlen_options(window_size=(-1, -1), softcap=0.0, alibi_slopes=None, deterministic=False,
+                    return_attn_probs=False, block_table=None, seqused_q=None, seqused_k=None,
+                    **kwargs):
+    """The options of ``flash_attn_varlen_func`` that ``_varlen`` takes; the
+    others are accepted and unused, as there."""
+    return dict(window_size=window_size, softcap=softcap, alibi_slopes=alibi_slopes,
+                return_attn_probs=return_attn_probs, block_table=block_table, seqused_q=seqused_q,
+                seqused_k=seqused_k)
 
 
 def flash_attn_varlen_kvpacked_func(q, kv, cu_seqlens_q, cu_seqlens_k, max_seqlen_q,
                                     max_seqlen_k, dropout_p=0.0, softmax_scale=None,
                                     causal=False, **kwargs):
     """Varlen with packed KV (reference :692-699). kv: (total_k, 2, nheads_k, headdim)."""
-    k, v = kv.unbind(dim=1)
-    return flash_attn_varlen_func(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q,
-                                  max_seqlen_k, dropout_p=dropout_p,
-                                  softmax_scale=softmax_scale, causal=causal, **kwargs)
+    k, v = unpack(kv, 1)
+    return _varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k,
+                   dropout_p=dropout_p, softmax_scale=softmax_scale, causal=causal, packed=2,
+                   **_varlen_options(**kwargs))
 
 
 def flash_attn_varlen_qkvpacked_func(qkv, cu_seqlens, max_seqlen, dropout_p=0.0,
                                      softmax_scale=None, causal=False, **kwargs):
     """Varlen with packed QKV (reference :702-708). qkv: (total, 3, nheads, headdim)."""
-    q, k, v = qkv.unbind(dim=1)
-    return flash_attn_varlen_func(q, k, v, cu_seqlens, cu_seqlens, max_seqlen, max_seqlen,
-                                  dropout_p=dropout_p, softmax_scale=softmax_scale,
-                                  causal=causal, **kwargs)
+    q, k, v = unpack(qkv, 1)
+    return _varlen(q, k, v, cu_seqlens, cu_seqlens, max_seqlen, max_seqlen, dropout_p=dropout_p,
+                   softmax_scale=softmax_scale, causal=causal, packed=3, **_varlen_options(**kwargs))
 
 
 class _AttentionModule(torch.nn.Module):

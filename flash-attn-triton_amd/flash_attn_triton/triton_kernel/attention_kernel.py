@@ -145,11 +145,64 @@ def _f32_alibi(alibi, device):
     return None if alibi is None else alibi.to(device=device, dtype=torch.float32).contiguous()
 
 
+class _Unpack(torch.autograd.Function):
+    """The q, k, v (or k, v) of a packed tensor along ``dim``, as views.  The
+    gradients come back as one packed tensor: in place where the backward wrote
+    them as slices of one (``_grad_buffers``), else stacked."""
+
+    @staticmethod
+    def forward(ctx, packed, dim):
+        ctx.dim = dim
+        return packed.unbind(dim)
+
+    @staticmethod
+    def backward(ctx, *grads):
+        g, n = grads[0], len(grads)
+        if g.ndim >= 3:
+            step = g.shape[-2] * g.shape[-1]
+            strides = [g.shape[-1], 1]
+            size = n * step
+            for extent in reversed(g.shape[:-2]):
+                strides.insert(0, size)
+                size *= extent
+            if (ctx.dim == g.ndim - 2 and list(g.stride()) == strides and all(
+                    x.stride() == g.stride() and x.shape == g.shape and x.dtype == g.dtype
+                    and x.untyped_storage().data_ptr() == g.untyped_storage().data_ptr()
+                    and x.storage_offset() == g.storage_offset() + i * step
+                    for i, x in enumerate(grads))):
+                shape = g.shape[:-2] + (n,) + g.shape[-2:]
+                return g.as_strided(shape, strides[:-2] + [step] + strides[-2:],
+                                    g.storage_offset()), None
+        return torch.stack(grads, ctx.dim), None
+
+
+def unpack(packed: torch.Tensor, dim: int):
+    """``packed.unbind(dim)`` whose gradient is not assembled by a copy when
+    the attention's backward can write the packed gradient itself (the callers
+    below take ``packed=`` the number of trailing tensors of q, k, v that come
+    from here)."""
+    return _Unpack.apply(packed, dim) if _needs_grad(packed) else packed.unbind(dim)
+
+
+def _grad_buffers(q, k, v, packed: int, zero: bool):
+    """Gradient tensors of q, k and v; the last ``packed`` of them (0, 2 or 3)
+    as slices of one tensor packed along the dim before the heads."""
+    make = torch.zeros if zero else torch.empty
+    ts = [q, k, v]
+    grads = [make(t.shape, dtype=t.dtype, device=t.device) for t in ts[:3 - packed]]
+    if packed:
+        t = ts[-1]
+        grads += make(t.shape[:-2] + (packed,) + t.shape[-2:], dtype=t.dtype,
+                      device=t.device).unbind(-3)
+    return grads
+
+
 def dense_backward(q, k, v, out, dout, lse, *, softmax_scale: float, causal: bool,
                    q_pos_offset: int = 0, window_left: int = -1, window_right: int = -1,
                    softcap: float = 0.0, alibi: Optional[torch.Tensor] = None,
                    dropout_p: float = 0.0, dropout_seed: int = 0,
-                   bias: Optional[torch.Tensor] = None, dbias: Optional[torch.Tensor] = None):
+                   bias: Optional[torch.Tensor] = None, dbias: Optional[torch.Tensor] = None,
+                   packed: int = 0):
     """Gradients ``(dq, dk, dv)`` of ``dense_forward`` from ``dout``, given its
     output and LSE (``fa_bwd_dense``).  Head dim 16 runs at 32 with zero padding
     (the extra dims contribute nothing to the scores and get zero gradients).
@@ -165,9 +218,7 @@ def dense_backward(q, k, v, out, dout, lse, *, softmax_scale: float, causal: boo
                                dbias=dbias)
         return tuple(g[..., :16] for g in grads)
     qk, kk, vk, ok, dok = (_kernel_ready(t) for t in (q, k, v, out, dout))
-    dq = torch.empty(q.shape, dtype=q.dtype, device=q.device)
-    dk = torch.empty(k.shape, dtype=k.dtype, device=k.device)
-    dv = torch.empty(v.shape, dtype=v.dtype, device=v.device)
+    dq, dk, dv = _grad_buffers(q, k, v, packed, zero=False)
     delta = torch.empty_like(lse)
     _native.bwd_dense(qk, kk, vk, ok, dok, lse, dq, dk, dv, delta, softmax_scale, causal,
                       q_pos_offset, window_left, window_right, softcap,
@@ -180,9 +231,10 @@ def varlen_backward(q, k, v, out, dout, lse, cu_q, cu_k, max_seqlen_q: int, max_
                     *, softmax_scale: float, causal: bool, window_left: int = -1,
                     window_right: int = -1, softcap: float = 0.0,
                     alibi: Optional[torch.Tensor] = None, dropout_p: float = 0.0,
-                    dropout_seed: int = 0):
+                    dropout_seed: int = 0, packed: int = 0, covered: bool = False):
     """Gradients ``(dq, dk, dv)`` of ``varlen_forward`` (``fa_bwd_varlen``).
-    Rows outside every sequence get zero gradients."""
+    Rows outside every sequence get zero gradients; ``covered`` states that the
+    sequences cover every row (the kernels then write all of them)."""
     if q.shape[-1] == 16:
         grads = varlen_backward(*(_pad_head_dim(t, 32) for t in (q, k, v, out, dout)), lse,
                                 cu_q, cu_k, max_seqlen_q, max_seqlen_k,
@@ -192,9 +244,7 @@ def varlen_backward(q, k, v, out, dout, lse, cu_q, cu_k, max_seqlen_q: int, max_
                                 dropout_seed=dropout_seed)
         return tuple(g[..., :16] for g in grads)
     qk, kk, vk, ok, dok = (_kernel_ready(t) for t in (q, k, v, out, dout))
-    dq = torch.zeros(q.shape, dtype=q.dtype, device=q.device)
-    dk = torch.zeros(k.shape, dtype=k.dtype, device=k.device)
-    dv = torch.zeros(v.shape, dtype=v.dtype, device=v.device)
+    dq, dk, dv = _grad_buffers(q, k, v, packed, zero=not covered)
     delta = torch.empty_like(lse)
     i32 = lambda t: t.to(device=q.device, dtype=torch.int32).contiguous()
     _native.bwd_varlen(qk, kk, vk, ok, dok, lse, dq, dk, dv, delta, i32(cu_q), i32(cu_k),
@@ -219,7 +269,7 @@ class _DenseAttention(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, q, k, v, softmax_scale, causal, q_pos_offset, window_left, window_right,
-                softcap, alibi, dropout_p, dropout_seed, bias4):
+                softcap, alibi, dropout_p, dropout_seed, bias4, packed):
         bias = None if bias4 is None else _expand_bias(bias4, q, k)
         out, lse = dense_forward(q, k, v, softmax_scale=softmax_scale, causal=causal,
                                  q_pos_offset=q_pos_offset, window_left=window_left,
@@ -228,14 +278,17 @@ class _DenseAttention(torch.autograd.Function):
                                  dropout_seed=dropout_seed)
         ctx.save_for_backward(q, k, v, out, lse, alibi, bias4)
         ctx.opts = (softmax_scale, causal, q_pos_offset, window_left, window_right, softcap,
-                    dropout_p, dropout_seed)
+                    dropout_p, dropout_seed, packed)
         ctx.mark_non_differentiable(lse)
+        ctx.set_materialize_grads(False)   # (no zero-filled gradient of the LSE)
         return out, lse
 
     @staticmethod
     def backward(ctx, dout, _dlse):
         q, k, v, out, lse, alibi, bias4 = ctx.saved_tensors
-        scale, causal, off, wl, wr, cap, dp, seed = ctx.opts
+        scale, causal, off, wl, wr, cap, dp, seed, packed = ctx.opts
+        if dout is None:
+            return (None,) * 14
         bias = dbias4 = dbias = None
         if bias4 is not None:
             bias = _expand_bias(bias4, q, k)
@@ -245,8 +298,8 @@ class _DenseAttention(torch.autograd.Function):
         dq, dk, dv = dense_backward(q, k, v, out, dout, lse, softmax_scale=scale, causal=causal,
                                     q_pos_offset=off, window_left=wl, window_right=wr,
                                     softcap=cap, alibi=alibi, dropout_p=dp, dropout_seed=seed,
-                                    bias=bias, dbias=dbias)
-        return (dq, dk, dv) + (None,) * 9 + (dbias4,)
+                                    bias=bias, dbias=dbias, packed=packed)
+        return (dq, dk, dv) + (None,) * 9 + (dbias4, None)
 
 
 class _VarlenAttention(torch.autograd.Function):
@@ -254,7 +307,8 @@ class _VarlenAttention(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, q, k, v, cu_q, cu_k, max_seqlen_q, max_seqlen_k, softmax_scale, causal,
-                window_left, window_right, softcap, alibi, dropout_p, dropout_seed, guard):
+                window_left, window_right, softcap, alibi, dropout_p, dropout_seed, guard, packed,
+                covered):
         out, lse = varlen_forward(q, k, v, cu_q, cu_k, max_seqlen_q, max_seqlen_k,
                                   softmax_scale=softmax_scale, causal=causal,
                                   window_left=window_left, window_right=window_right,
@@ -262,29 +316,32 @@ class _VarlenAttention(torch.autograd.Function):
                                   dropout_p=dropout_p, dropout_seed=dropout_seed, guard=guard)
         ctx.save_for_backward(q, k, v, out, lse, cu_q, cu_k, alibi)
         ctx.opts = (max_seqlen_q, max_seqlen_k, softmax_scale, causal, window_left,
-                    window_right, softcap, dropout_p, dropout_seed)
+                    window_right, softcap, dropout_p, dropout_seed, packed, covered)
         ctx.mark_non_differentiable(lse)
+        ctx.set_materialize_grads(False)   # (no zero-filled gradient of the LSE)
         return out, lse
 
     @staticmethod
     def backward(ctx, dout, _dlse):
         q, k, v, out, lse, cu_q, cu_k, alibi = ctx.saved_tensors
-        mq, mk, scale, causal, wl, wr, cap, dp, seed = ctx.opts
+        mq, mk, scale, causal, wl, wr, cap, dp, seed, packed, covered = ctx.opts
+        if dout is None:
+            return (None,) * 18
         dq, dk, dv = varlen_backward(q, k, v, out, dout, lse, cu_q, cu_k, mq, mk,
                                      softmax_scale=scale, causal=causal, window_left=wl,
                                      window_right=wr, softcap=cap, alibi=alibi, dropout_p=dp,
-                                     dropout_seed=seed)
-        return (dq, dk, dv) + (None,) * 13
+                                     dropout_seed=seed, packed=packed, covered=covered)
+        return (dq, dk, dv) + (None,) * 15
 
 
 def dense_attention(q, k, v, *, softmax_scale: float, causal: bool, q_pos_offset: int = 0,
                     window_left: int = -1, window_right: int = -1, softcap: float = 0.0,
                     alibi: Optional[torch.Tensor] = None, return_lse: bool = False,
                     bias: Optional[torch.Tensor] = None, dropout_p: float = 0.0,
-                    dropout_seed: int = 0):
+                    dropout_seed: int = 0, packed: int = 0):
     """``dense_forward`` that is differentiable in q, k, v and ``bias`` (fp16 /
     bf16).  ``bias`` (optional) is a 4-D fp32 tensor that broadcasts to the
-    ``[B, Hq, Sq, Sk]`` scores."""
+    ``[B, Hq, Sq, Sk]`` scores.  ``packed``: see ``unpack``."""
     if not _needs_grad(q, k, v, bias):
         res = dense_forward(q, k, v, softmax_scale=softmax_scale, causal=causal,
                             q_pos_offset=q_pos_offset, window_left=window_left,
@@ -294,7 +351,8 @@ def dense_attention(q, k, v, *, softmax_scale: float, causal: bool, q_pos_offset
                             dropout_p=dropout_p, dropout_seed=dropout_seed)
         return res
     out, lse = _DenseAttention.apply(q, k, v, softmax_scale, causal, q_pos_offset, window_left,
-                                     window_right, softcap, alibi, dropout_p, dropout_seed, bias)
+                                     window_right, softcap, alibi, dropout_p, dropout_seed, bias,
+                                     packed)
     return (out, lse) if return_lse else out
 
 
@@ -303,8 +361,10 @@ def varlen_attention(q, k, v, cu_q, cu_k, max_seqlen_q: int, max_seqlen_k: int, 
                      window_right: int = -1, softcap: float = 0.0,
                      alibi: Optional[torch.Tensor] = None, return_lse: bool = False,
                      dropout_p: float = 0.0, dropout_seed: int = 0,
-                     guard: Optional[torch.Tensor] = None):
-    """``varlen_forward`` that is differentiable in q, k, v (fp16 / bf16)."""
+                     guard: Optional[torch.Tensor] = None, packed: int = 0,
+                     covered: bool = False):
+    """``varlen_forward`` that is differentiable in q, k, v (fp16 / bf16).
+    ``packed``: see ``unpack``; ``covered``: see ``varlen_backward``."""
     if not _needs_grad(q, k, v):
         return varlen_forward(q, k, v, cu_q, cu_k, max_seqlen_q, max_seqlen_k,
                               softmax_scale=softmax_scale, causal=causal,
@@ -313,7 +373,7 @@ def varlen_attention(q, k, v, cu_q, cu_k, max_seqlen_q: int, max_seqlen_k: int, 
                               dropout_p=dropout_p, dropout_seed=dropout_seed, guard=guard)
     out, lse = _VarlenAttention.apply(q, k, v, cu_q, cu_k, max_seqlen_q, max_seqlen_k,
                                       softmax_scale, causal, window_left, window_right, softcap,
-                                      alibi, dropout_p, dropout_seed, guard)
+                                      alibi, dropout_p, dropout_seed, guard, packed, covered)
     return (out, lse) if return_lse else out
 
 
