@@ -1,6 +1,6 @@
 // fp32 attention forward for gfx950: dense / cross / varlen prefill and the
 // KV-cache path, for fp32 q/k/v (flash_attn_interface.py:95-96 accepts fp16 and
-// fp32; BASELINE config 1 is fp32).
+// fp32).
 //
 // The reference runs its Triton kernels on fp32 tensors with fp32 dot products
 // and keeps P in the input dtype for the PV product

@@ -36,10 +36,11 @@ hipError_t launch_fwd_cfg(FwdParams p, int rows_for_grid, int outer_blocks, hipS
 
 // Prefill tile table (fa_prefill_kernel.h), keyed by head dim and by whether
 // the problem is masked (causal, window or varlen):
-//   D = 128, masked  : 4 waves, 32-key tiles, 3 waves per SIMD (165 VGPRs);
-//                      with the generic epilogue 2 waves, 2 per SIMD, tiles
-//                      by LDS-DMA through a 3 K / 2 V stage ring (KS = 3)
-//   D = 128, unmasked: 8 waves (256 query rows share each K/V tile), 64-key tiles
+//   D = 128          : the generic epilogue only (fa_prefill_pp.h and
+//                      fa_prefill_persist.h have the plain one); masked 2 waves,
+//                      2 per SIMD, tiles by LDS-DMA through a 3 K / 2 V stage
+//                      ring (KS = 3); unmasked 8 waves (256 query rows share
+//                      each K/V tile), 64-key tiles
 //   D = 256          : 8 waves, 32-key tiles (the O^T accumulators take 128 VGPRs)
 //   D = 32 / 64      : 4 waves, 64-key tiles (64 with the generic epilogue or
 //                      attn_bias only: fa_prefill_d64.h has the plain one)
@@ -196,33 +197,31 @@ hipError_t launch_prefill(const FwdParams& p, hipStream_t st) {
   }
   const bool masked = p.causal || p.window_left >= 0 || p.window_right >= 0 || p.cu_q != nullptr;
   if constexpr (D == 128) {
-    // The generic epilogue stays on prefill_kernel: measured at BASELINE
-    // config 5 (varlen, causal + window 1024, ALiBi, softcap) the ping-pong
-    // kernel is 1.22x slower there (its 256-row blocks visit every key tile
-    // of the block's window for all rows, and the softmax phase outgrows the
-    // GEMM phase).
+    // The generic epilogue stays on prefill_kernel: measured on 32 sequences
+    // of 128 to 4096 tokens (H16, causal + window 1024, ALiBi, softcap) the
+    // ping-pong kernel is 1.22x slower (its 256-row blocks visit every key
+    // tile of the block's window for all rows, and the softmax phase outgrows
+    // the GEMM phase).
     if constexpr (!GEN) {
       if (p.cu_q != nullptr) return launch_prefill_pp<T, D, kPpVarlen, false>(p, st);
       bool launched = false;
       hipError_t e = launch_prefill_persist<T, D>(p, st, &launched);
       if (e != hipSuccess || launched) return e;
       return launch_prefill_pp<T, D, kPpDense, false>(p, st);
+    } else {
+      // The generic epilogue (varlen, ALiBi, softcap, window) does not fit the
+      // 168-VGPR budget of 3 waves per SIMD without spilling: 2 waves, in
+      // workgroups of 2 (64 rows; measured on the sequences above with the
+      // tiles staged through VGPRs: 4 % faster than 4-wave workgroups, which
+      // visit more key tiles per row at a window edge; 3 waves per SIMD spill
+      // and were 3.3x slower, 64-key tiles 1.6x).
+      // The tiles go global -> LDS by LDS-DMA in a ring of 3 K and 2 V stages
+      // (40 KiB: four workgroups per CU).  Measured there on one MI355X:
+      // 884 us against 927 us with the tiles staged through VGPRs; the 4-wave
+      // form with 5 + 4 stages measured 927 us.
+      if (masked) return launch_prefill_cfg<T, D, 2, 32, true, 2, false, 3>(p, st);
+      return launch_prefill_cfg<T, D, 8, 64, true, 2>(p, st);
     }
-    // The generic epilogue (varlen, ALiBi, softcap, window) does not fit the
-    // 168-VGPR budget of 3 waves per SIMD without spilling: 2 waves, in
-    // workgroups of 2 (64 rows; measured at BASELINE config 5 with the tiles
-    // staged through VGPRs: 4 % faster than 4-wave workgroups, which visit
-    // more key tiles per row at a window edge; 3 waves per SIMD spill and
-    // were 3.3x slower, 64-key tiles 1.6x).
-    // The tiles go global -> LDS by LDS-DMA in a ring of 3 K and 2 V stages
-    // (40 KiB: four workgroups per CU).  Measured at BASELINE config 5 on one
-    // MI355X: 884 us against 927 us with the tiles staged through VGPRs; the
-    // 4-wave form with 5 + 4 stages measured 927 us.
-    if (masked) {
-      if constexpr (GEN) return launch_prefill_cfg<T, D, 2, 32, GEN, 2, false, 3>(p, st);
-      else return launch_prefill_cfg<T, D, 4, 32, GEN, 3>(p, st);
-    }
-    return launch_prefill_cfg<T, D, 8, 64, GEN, 2>(p, st);
   } else if constexpr (D == 256) {
     return launch_prefill_cfg<T, D, 8, 32, GEN, 2>(p, st);
   } else if constexpr (D == 64) {

@@ -37,12 +37,13 @@
 // tiles downwards, from the last visible one: with ALiBi (and with the
 // recency typical of real attention) scores grow towards the diagonal, and
 // walking upwards the running max moved past the rescale slack on about
-// 40 % of the tiles at BASELINE config 5 (64 multiplies of O^T each);
+// 40 % of the tiles of 32 sequences of 128 to 4096 tokens (H16, window 1024,
+// ALiBi, softcap; 64 multiplies of O^T each);
 // downwards the first tiles set it (measured 1 % faster there).  The tile
 // loads step running 64-bit bases and ring slots instead of forming each
 // tile's address from its index: the 64-bit products and slot divisions were
-// about 40 scalar instructions per tile, and dropping them made BASELINE
-// config 5 3 % faster (848 -> 822 us per launch on one MI355X).
+// about 40 scalar instructions per tile, and dropping them made that launch
+// 3 % faster (848 -> 822 us on one MI355X).
 #pragma once
 
 #include "fa_fwd_kernel.h"
@@ -718,7 +719,7 @@ void prefill_kernel(const FwdParams p) {
     // The output goes through LDS (the tile area, once every wave's last
     // tile reads are done) and out as whole rows: stored straight from the
     // accumulators, each instruction wrote 8 bytes of 32 rows, and the
-    // partial lines reached HBM piecemeal (measured at BASELINE config 5:
+    // partial lines reached HBM piecemeal (measured on those sequences:
     // 290.6 MB written for a 134.2 MB output).
     static_assert(NW * kStageOutBytes <= prefill_lds_bytes<D, NW, BN, KS>(),
                   "output staging must fit the tile area");

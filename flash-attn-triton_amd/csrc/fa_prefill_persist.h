@@ -421,8 +421,8 @@ void prefill_persist_kernel(const FwdParams p) {
   // Running tile bases of the plain phases (non-causal): the plain phase of
   // tile j loads K_{j+3} and V_{j+2} of the current block, so each base steps
   // one tile per phase (set at the block's start) instead of being formed
-  // from j: ten scalar instructions fewer per softmax phase, 0.8 % at BASELINE
-  // config 2 non-causal.  The causal kernel keeps the indexed form: the two
+  // from j: ten scalar instructions fewer per softmax phase, 0.8 % at B4
+  // H32 S4096 non-causal.  The causal kernel keeps the indexed form: the two
   // running bases there raised its scalar-register spills from 16 to 27 and
   // it ran no faster.
   const uint16_t* k_run = kg;
