@@ -70,6 +70,12 @@ def _host_minmax(a: torch.Tensor, b: Optional[torch.Tensor], diff: bool):
     return int(x.min()), int(x.max())
 
 
+def _outside(item, got) -> bool:
+    """Whether the (min, max) of a queued range check leaves its bounds."""
+    _, _, lo, hi, _ = item
+    return (lo is not None and got[0] < lo) or (hi is not None and got[1] > hi)
+
+
 class Deferred:
     def __init__(self, side: bool = False) -> None:
         # (kind, exception or None, lo, hi, payload), in queue order:
@@ -142,9 +148,10 @@ class Deferred:
         ``side=True`` the range checks reduce on a second stream, so the
         launch does not queue behind them.  Only kernels that stay inside
         their buffers whatever the checked arrays hold may be launched this
-        way, or, with ``guarded`` (``ranges_only()`` must hold), kernels that
-        return at once when one of the int32 device flags ``launch(flags)``
-        gets is set (None: nothing was checked on the device)."""
+        way, or, with ``guarded`` (range checks only), kernels that return at
+        once when one of the int32 device flags ``launch(flags)`` gets is set
+        (None: nothing was checked on the device).  Checks of host tensors have
+        no flag: when one of them fails, a guarded launch is not made."""
         items, self._items = self._items, []
         self._nvalues = 0
         if not items:
@@ -210,6 +217,9 @@ class Deferred:
             else:
                 words = packed.tolist()
         failed = None
+        # (`results` holds the host tensors' ranges so far.)
+        if guarded and any(_outside(items[i], r) for i, r in results.items()):
+            launch = None
         if launch is not None:
             try:
                 launch(guard) if guarded else launch()
@@ -236,10 +246,9 @@ class Deferred:
             scalars_dec.append(_decode(words[pos:pos + n], dt))
             pos += n
         values, k = [], 0
-        for i, (kind, exc, lo, hi, _) in enumerate(items):
+        for i, (kind, exc, _, _, _) in enumerate(items):
             if kind == "range":
-                mn, mx = results[i]
-                if (lo is not None and mn < lo) or (hi is not None and mx > hi):
+                if _outside(items[i], results[i]):
                     raise exc
             elif kind == "minmax":
                 values.append(results[i])

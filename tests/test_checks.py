@@ -69,3 +69,20 @@ def test_adjacent_difference_ranges_and_value_ranges(dtype):
     with pytest.raises(ValueError, match="fit"):
         chk.flush()
     assert (i, j) == (0, 1)
+
+
+@pytest.mark.parametrize("bad", [None, 0, 1])
+def test_failing_host_check_stops_a_guarded_launch(bad):
+    # Host tensors have no device flag to guard a launch with: a guarded launch goes out only if their checks pass;
+    # an unguarded one (safe on any values) goes out first, and the check still raises.
+    for guarded in (True, False):
+        chk, launched = Deferred(), []
+        chk.check_range(torch.tensor([1, 2]), 0, 1 if bad == 0 else 2, ValueError("first"))
+        chk.check_range(torch.tensor([7, 3]), 4 if bad == 1 else 0, None, IndexError("second"))
+        call = lambda *flags: launched.append(flags)
+        if bad is None:
+            assert chk.flush(call, guarded=guarded) == []
+        else:
+            with pytest.raises((ValueError, IndexError)[bad], match=("first", "second")[bad]):
+                chk.flush(call, guarded=guarded)
+        assert launched == ([] if guarded and bad is not None else [(None,) if guarded else ()])

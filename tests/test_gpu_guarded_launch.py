@@ -30,16 +30,16 @@ def _tables(rows, dtype):
     return ang.cos().to(dtype), ang.sin().to(dtype)
 
 
-@pytest.mark.parametrize("what", ["length", "negative", "page", "rotary", "leftpad"])
+@pytest.mark.parametrize("what", ["length", "negative", "page", "host_page", "rotary", "leftpad"])
 def test_rejected_append_leaves_the_cache(what):
     from flash_attn_triton import flash_attn_with_kvcache
-    a = _append_args(paged=what == "page")
+    a = _append_args(paged=what in ("page", "host_page"))
     exc, match = ValueError, "do not fit"
     if what == "length":
         a["cache_seqlens"][1] = 255
     elif what == "negative":
         a["cache_seqlens"][0] = -1
-    elif what == "page":
+    elif what in ("page", "host_page"):
         a["block_table"][2, 3] = 12
         exc, match = ValueError, "invalid physical page"
     elif what == "rotary":
@@ -47,7 +47,8 @@ def test_rejected_append_leaves_the_cache(what):
         exc, match = IndexError, "rotary"
     else:
         a["cache_leftpad"] = torch.tensor([0, 3, 1], dtype=torch.int32)
-    d = {n: t.to(DEV) for n, t in a.items()}
+    # (host_page: a block table on the CPU, which is checked there)
+    d = {n: t if what == "host_page" and n == "block_table" else t.to(DEV) for n, t in a.items()}
     for _ in range(2):
         with pytest.raises(exc, match=match):
             flash_attn_with_kvcache(**d, causal=True)
