@@ -68,6 +68,18 @@ __device__ inline void wait_loads() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
+// Ring step barrier: at most N tile loads of this wave are outstanding, and
+// every LDS read it has issued has returned, so that after it any wave may
+// refill what was read.  (The products that use the reads are not memory
+// operations: without the scheduling barriers nothing keeps them, and with
+// them the compiler's own wait, on this side of the barrier.)
+template <int N>
+__device__ inline void ring_barrier() {
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
 // MODE: kPpDense / kPpVarlen / kPpCache (fa_prefill_pp.h).
 template <class T, int MODE, bool PAGED>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3)))
@@ -430,11 +442,10 @@ void prefill_d64_kernel(const FwdParams p) {
   // ------------------------------------------------------------ main loop
   // Top of step it: this wave's loads of its tile have landed once at most
   // those of step it + 1 are outstanding; the barrier makes everyone's
-  // visible, and every wave is done with step it - 1, whose slot the loads of
-  // step it + 2 refill.
+  // visible, and every wave has its reads of step it - 1, whose slot the loads
+  // of step it + 2 refill.
   auto top = [&](int it, int refill) __attribute__((always_inline)) {
-    wait_loads<2 * IPW>();
-    asm volatile("s_barrier" ::: "memory");
+    ring_barrier<2 * IPW>();
     issue(it + 2, refill);
   };
   // After a step: the block-table entry the next step's loads need, in flight
