@@ -38,7 +38,8 @@ hipError_t launch_dkdv(BwdParams p, hipStream_t st) {
   if (total > 0x7fffffff) return hipErrorInvalidConfiguration;
   if (total <= 0) return hipSuccess;
   p.total_blocks = (int)total;
-  p.span = l2_span(p.seqlen_q, D, p.group, 1, VARLEN ? 1 : 2);
+  p.span = VARLEN ? kv_rr_span(p.seqlen_q, D, p.group, (int64_t)p.heads_k * p.batch)
+                  : l2_span(p.seqlen_q, D, p.group, 1, 2);
   hipLaunchKernelGGL(kern, dim3((unsigned)total), dim3(Tile::NT), (unsigned)lds, st, p);
   return hipGetLastError();
 }
@@ -65,7 +66,8 @@ hipError_t launch_dkdv_split_st(BwdParams p, hipStream_t st) {
   if (total > 0x7fffffff) return hipErrorInvalidConfiguration;
   if (total <= 0) return hipSuccess;
   p.total_blocks = (int)total;
-  p.span = l2_span(p.seqlen_q, D, p.group, 1, VARLEN ? 1 : 2);
+  p.span = VARLEN ? kv_rr_span(p.seqlen_q, D, p.group, (int64_t)p.heads_k * p.batch)
+                  : l2_span(p.seqlen_q, D, p.group, 1, 2);
   hipLaunchKernelGGL(kern, dim3((unsigned)total), dim3(Tile::NT), (unsigned)lds, st, p);
   return hipGetLastError();
 }
@@ -105,7 +107,8 @@ hipError_t launch_bwd_v(BwdParams p, hipStream_t st) {
       p.total_blocks = (int)total;
       // (query heads of one K/V head share its tiles; the varlen order counts
       // K/V heads)
-      p.span = l2_span(p.seqlen_k, D, 1, VARLEN ? 1 : p.group, VARLEN ? 1 : 2);
+      p.span = VARLEN ? kv_rr_span(p.seqlen_k, D, 1, (int64_t)p.heads_k * p.batch)
+                      : l2_span(p.seqlen_k, D, 1, p.group, 2);
       hipLaunchKernelGGL(kern, dim3((unsigned)total), dim3(Tile::NT), Tile::LDS_BYTES, st, p);
       e = hipGetLastError();
       if (e != hipSuccess) return e;

@@ -178,7 +178,8 @@ __device__ inline void work_item(int L, int total, int n_mblocks, bool heavy_fir
 // heads interleaved, the last first when heavy_first).  The last n_kv % 8 K/V
 // heads, if any, follow with their items spread over all XCDs.
 // Returns false (no item assigned) unless total = n_kv * group * n_mblocks.
-__device__ inline bool work_item_kv_rr(int L, int total, int n_mblocks, int group,
+// span is at most n_kv (kv_rr_span), which keeps span * per_kv within total.
+__host__ __device__ inline bool work_item_kv_rr(int L, int total, int n_mblocks, int group,
                                        bool heavy_first, int span, int& mb, int& grp) {
   constexpr int kXcds = 8;
   const int per_kv = group * n_mblocks;   // items per K/V head
@@ -187,7 +188,8 @@ __device__ inline bool work_item_kv_rr(int L, int total, int n_mblocks, int grou
   const bool main = L < heads * kXcds * per_kv;
   const int k = main ? L / kXcds : L - heads * kXcds * per_kv;
   const int k0 = k / (span * per_kv) * span;   // this span's first round (tail: first head)
-  const int cw = min(span, (main ? heads : total / per_kv - heads * kXcds) - k0);
+  const int left = (main ? heads : total / per_kv - heads * kXcds) - k0;
+  const int cw = span < left ? span : left;
   int r = k - k0 * per_kv;
   mb = r / (group * cw);
   r -= mb * group * cw;
@@ -257,6 +259,14 @@ inline int l2_span(int64_t rows, int64_t head_dim, int64_t heads_streamed, int64
   const int64_t bytes = 4 * (rows > 0 ? rows : 1) * head_dim * heads_streamed;   // both tensors
   const int64_t n = (int64_t(4) << 20) * heads_sharing / bytes;
   return (int)(n < least ? least : n > 4096 ? 4096 : n);
+}
+// The same for work_item_kv_rr, in a launch of n_kv K/V heads.  A span past all
+// of them orders the items as n_kv does, and short keys against long queries
+// of many heads (or the reverse, in the backward) would take its product with
+// a head's items past 2^31.
+inline int kv_rr_span(int64_t rows, int64_t head_dim, int64_t heads_streamed, int64_t n_kv) {
+  const int n = l2_span(rows, head_dim, heads_streamed, 1, 1);
+  return n_kv < n ? (int)(n_kv > 1 ? n_kv : 1) : n;
 }
 
 __device__ inline u32x4 load16(const void* p) { return *reinterpret_cast<const u32x4*>(p); }

@@ -81,7 +81,7 @@ hipError_t launch_prefill_pp(FwdParams p, hipStream_t st) {
   if (total <= 0) return hipSuccess;
   if (total > 0x7fffffff) return hipErrorInvalidConfiguration;
   p.total_blocks = (int)total;
-  p.span = l2_span(p.seqlen_k, D, 1, 1, 1);   // (varlen)
+  if (MODE == kPpVarlen) p.span = kv_rr_span(p.seqlen_k, D, 1, (int64_t)p.heads_k * p.batch);
   hipLaunchKernelGGL(kern, dim3((unsigned)total), dim3(Tile::NT), Tile::LDS_BYTES, st, p);
   return hipGetLastError();
 }
@@ -179,7 +179,7 @@ hipError_t launch_prefill_d64(FwdParams p, hipStream_t st) {
   if (total <= 0) return hipSuccess;
   if (total > 0x7fffffff) return hipErrorInvalidConfiguration;
   p.total_blocks = (int)total;
-  p.span = MODE == kPpVarlen ? l2_span(p.seqlen_k, 64, 1, 1, 1)
+  p.span = MODE == kPpVarlen ? kv_rr_span(p.seqlen_k, 64, 1, (int64_t)p.heads_k * p.batch)
                              : p.seqlen_k > 0 && p.seqlen_k < 4096 ? 32768 / p.seqlen_k : 8;
   hipLaunchKernelGGL(kern, dim3((unsigned)total), dim3(Tile::NT), Tile::LDS_BYTES, st, p);
   return hipGetLastError();
