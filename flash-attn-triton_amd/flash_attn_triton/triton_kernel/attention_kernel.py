@@ -287,8 +287,8 @@ class _DenseAttention(torch.autograd.Function):
     def backward(ctx, dout, _dlse):
         q, k, v, out, lse, alibi, bias4 = ctx.saved_tensors
         scale, causal, off, wl, wr, cap, dp, seed, packed = ctx.opts
-        if dout is None:
-            return (None,) * 14
+        if dout is None:   # no gradient reaches the output: the inputs' are zeros
+            dout = torch.zeros_like(out)
         bias = dbias4 = dbias = None
         if bias4 is not None:
             bias = _expand_bias(bias4, q, k)
@@ -325,8 +325,8 @@ class _VarlenAttention(torch.autograd.Function):
     def backward(ctx, dout, _dlse):
         q, k, v, out, lse, cu_q, cu_k, alibi = ctx.saved_tensors
         mq, mk, scale, causal, wl, wr, cap, dp, seed, packed, covered = ctx.opts
-        if dout is None:
-            return (None,) * 18
+        if dout is None:   # no gradient reaches the output: the inputs' are zeros
+            dout = torch.zeros_like(out)
         dq, dk, dv = varlen_backward(q, k, v, out, dout, lse, cu_q, cu_k, mq, mk,
                                      softmax_scale=scale, causal=causal, window_left=wl,
                                      window_right=wr, softcap=cap, alibi=alibi, dropout_p=dp,
