@@ -820,7 +820,8 @@ int fa_kvcache_update(const void* k_new, const void* v_new, void* k_cache, void*
   if (!cache_seqlens || (n_new > 0 && (!k_new || !v_new || !k_cache || !v_cache || !k_new_stride ||
                                        !v_new_stride || !k_cache_stride || !v_cache_stride)))
     return fail(FA_ERR_INVALID, "%s: null pointer argument", name);
-  if ((rotary_cos == nullptr) != (rotary_sin == nullptr) ||
+  // (q_out without tables, which an empty table is too, would stay unwritten.)
+  if ((rotary_cos == nullptr) != (rotary_sin == nullptr) || (!rotary_cos && q_out) ||
       (rotary_cos && (!q || !q_out || !q_stride || !q_out_stride)))
     return fail(FA_ERR_INVALID, "%s: rotary_cos, rotary_sin, q and q_out go together", name);
   if (!supported_dtype(dtype) || (rotary_cos && !supported_dtype(table_dtype)))

@@ -361,8 +361,8 @@ int fa_rotary_q(const void* q, void* out, const int32_t* cache_seqlens,
                 const int64_t* out_stride, int dtype, fa_stream_t stream);
 
 /* The append of fa_kvcache_append and the query rotation of fa_rotary_q in one
- * launch: n_new may be 0 (no append) and rotary_cos NULL (no rotation).  The
- * tables are [rotary_rows, rotary_dim / 2] contiguous of table_dtype, rounded
+ * launch: n_new may be 0 (no append) and rotary_cos NULL (no rotation; q_out
+ * is then NULL too).  The tables are [rotary_rows, rotary_dim / 2] contiguous of table_dtype, rounded
  * to `dtype` as they are read.  cache_seqlens holds the lengths before the
  * append; lens_out (nullable, int32 [batch]) receives them plus n_new, and the
  * queries are rotated at those.  With a failed guard (see fa_check_bounds)

@@ -110,6 +110,19 @@ def test_dense_rejects_unsupported_dtype_and_head_dim(lib):
     assert status == _native.FA_ERR_UNSUPPORTED
 
 
+def test_kvcache_update_rejects_a_rotation_without_tables(lib):
+    # Tables without columns have no address: the rotated queries would stay unwritten.
+    st = _native._strides((1024, 64, 64))
+    one = ctypes.c_void_p(16)   # never dereferenced
+    def update(cos, q_out):
+        return lib.fa_kvcache_update(None, None, None, None, one, None, 0, 0, 0, None, 1, None, 64, cos, cos, 0, 64, 64,
+                                     1, one, q_out, 1, 2, None, 1, 0, 2, 64, None, None, None, None, st, st, 0, None, 0,
+                                     None)
+    assert update(None, one) == _native.FA_ERR_INVALID and b"go together" in lib.fa_last_error_string()
+    assert update(one, None) == _native.FA_ERR_INVALID
+    assert update(None, None) == 0   # nothing to append or rotate
+
+
 def test_python_api_validation_on_cpu():
     """Checks the reference runs before any launch (flash_attn_interface.py:96-127)."""
     from flash_attn_triton import flash_attn_func, flash_attn_varlen_func
