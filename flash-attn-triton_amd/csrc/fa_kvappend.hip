@@ -22,6 +22,7 @@
 // One thread per output element.  Out-of-range slots, pages or table rows
 // (which the Python layer rejects before calling) are skipped, never read or
 // written.
+#include <algorithm>
 #include <type_traits>
 
 #include "fa_common.h"
@@ -181,9 +182,10 @@ hipError_t fa_launch_kv_update(int dtype, const fa::UpdateParams& p, hipStream_t
   const int64_t kv = (int64_t)p.a.batch * p.a.n_new * p.a.heads_k * p.a.head_dim;
   const int64_t qn = p.cos != nullptr ? (int64_t)p.q.batch * p.q.seqlen_q * p.q.heads * p.q.head_dim : 0;
   const int64_t nk = (kv + 255) / 256, nq = (qn + 255) / 256;
-  if (nk + nq <= 0) return hipSuccess;
-  if (nk + nq > 0x7fffffff) return hipErrorInvalidConfiguration;
-  const dim3 grid((unsigned)(nk + nq));
+  const int64_t blocks = std::max(nk + nq, (int64_t)(p.lens_out != nullptr && p.a.batch > 0));
+  if (blocks <= 0) return hipSuccess;
+  if (blocks > 0x7fffffff) return hipErrorInvalidConfiguration;
+  const dim3 grid((unsigned)blocks);
   if (dtype == 0) hipLaunchKernelGGL(fa::kv_update_kernel<fa::F16>, grid, dim3(256), 0, st, p, (int)nk);
   else if (dtype == 1) hipLaunchKernelGGL(fa::kv_update_kernel<fa::BF16>, grid, dim3(256), 0, st, p, (int)nk);
   else hipLaunchKernelGGL(fa::kv_update_kernel<float>, grid, dim3(256), 0, st, p, (int)nk);

@@ -362,11 +362,11 @@ int fa_rotary_q(const void* q, void* out, const int32_t* cache_seqlens,
 
 /* The append of fa_kvcache_append and the query rotation of fa_rotary_q in one
  * launch: n_new may be 0 (no append) and rotary_cos NULL (no rotation; q_out
- * is then NULL too).  The tables are [rotary_rows, rotary_dim / 2] contiguous of table_dtype, rounded
- * to `dtype` as they are read.  cache_seqlens holds the lengths before the
- * append; lens_out (nullable, int32 [batch]) receives them plus n_new, and the
- * queries are rotated at those.  With a failed guard (see fa_check_bounds)
- * nothing is written. */
+ * is then NULL too).  The tables are [rotary_rows, rotary_dim / 2] contiguous
+ * of table_dtype, rounded to `dtype` as they are read.  cache_seqlens holds
+ * the lengths before the append; lens_out (nullable, int32 [batch]) receives
+ * them plus n_new, and the queries are rotated at those.  With a failed guard
+ * (see fa_check_bounds) nothing is written. */
 int fa_kvcache_update(const void* k_new, const void* v_new, void* k_cache, void* v_cache,
                       const int32_t* cache_seqlens, const int32_t* block_table,
                       int64_t block_table_stride, int64_t page_size, int64_t num_pages,

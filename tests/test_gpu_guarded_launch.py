@@ -149,3 +149,16 @@ def test_check_behind_queued_work_and_launch_errors():
     chk.check_range(lens, 0, 1000, ValueError("check"))
     with pytest.raises(KeyError):
         chk.flush(fails)
+
+
+def test_update_writes_lengths_without_work():
+    # Nothing to append or rotate: the new lengths are written all the same, except with a failed guard.
+    from flash_attn_triton import _native
+    kc, q = torch.zeros((3, 16, 2, D), dtype=torch.float16, device=DEV), torch.zeros((3, 1, 2, D), dtype=torch.float16,
+                                                                                   device=DEV)
+    lens = torch.tensor([5, 0, 16], dtype=torch.int32, device=DEV)
+    for flag in (0, 1):
+        out = torch.full((3,), -7, dtype=torch.int32, device=DEV)
+        guard = torch.tensor([0, flag], dtype=torch.int32, device=DEV)
+        _native.kvcache_update(None, None, kc, kc, lens, None, None, None, 16, None, None, True, q, None, out, guard)
+        assert out.tolist() == ([-7] * 3 if flag else [5, 0, 16])
