@@ -137,21 +137,27 @@ inline bool pp_pages(const FwdParams& p, int head_dim) {
   return p.block_table != nullptr && p.page_size % (head_dim == 64 ? 16 : 8) == 0;
 }
 
+// Row strides (elements) whose offsets from a wave's or tile's first row stay
+// far inside the 32 bits of a buffer load's offset.  The forms below take no
+// others; the kernels they replaced address each row in 64 bits, the queries'
+// at head dim 64 and every row of the KV-cache and paged ones.
+constexpr int64_t kMaxRowStride = (int64_t)1 << 24;
+inline bool row_strides_fit(const FwdParams& p) {
+  return p.q_ss <= kMaxRowStride && p.k_ss <= kMaxRowStride && p.v_ss <= kMaxRowStride;
+}
+
 // KV-cache launches that run on the ping-pong kernel (head dim 128) or
 // prefill_d64_kernel (64) instead of fwd_kernel: more rows than the decode
-// kernel's 32, pages as above, strides whose 32-row offsets stay far inside 32
-// bits, and neither ALiBi nor a scale <= 0 (`generic`).  Ahead over the whole of that range:
-// per call with fwd_kernel and with it, bf16, MI355X, 512 queries and 32 / 8
-// heads 614 -> 168 us; 33 rows per KV head (the fewest; 32 KV heads, B8) 515 ->
-// 192 us; 64 queries (B4) 135 -> 102 us, where the host's argument checks bound
-// both.
+// kernel's 32, pages and strides as above, and neither ALiBi nor a scale <= 0
+// (`generic`).  Ahead over the whole of that range: per call with fwd_kernel
+// and with it, bf16, MI355X, 512 queries and 32 / 8 heads 614 -> 168 us; 33
+// rows per KV head (the fewest; 32 KV heads, B8) 515 -> 192 us; 64 queries
+// (B4) 135 -> 102 us, where the host's argument checks bound both.
 inline bool cache_pp_route(const FwdParams& p, int head_dim, bool generic) {
-  constexpr int64_t kMaxStride = (int64_t)1 << 24;   // elements
   const int64_t rows = (int64_t)p.seqlen_q * p.group;
   return (head_dim == 128 || head_dim == 64) && !generic && rows > 32 &&
-         (p.block_table == nullptr || pp_pages(p, head_dim)) &&
-         p.q_ss <= kMaxStride && p.q_sh * p.group <= kMaxStride && p.k_ss <= kMaxStride &&
-         p.v_ss <= kMaxStride;
+         (p.block_table == nullptr || pp_pages(p, head_dim)) && row_strides_fit(p) &&
+         p.q_sh * p.group <= kMaxRowStride;
 }
 
 // Head dim 64, plain epilogue (fa_prefill_d64.h): 4 waves, 128 rows per
@@ -226,11 +232,12 @@ hipError_t launch_prefill(const FwdParams& p, hipStream_t st) {
     return launch_prefill_cfg<T, D, 8, 32, GEN, 2>(p, st);
   } else if constexpr (D == 64) {
     if constexpr (!GEN) {
-      if (p.cu_q != nullptr) return launch_prefill_d64<T, kPpVarlen, false>(p, st);
-      return launch_prefill_d64<T, kPpDense, false>(p, st);
-    } else {
-      return launch_prefill_cfg<T, D, 4, 64, GEN, 2>(p, st);
+      if (p.q_ss <= kMaxRowStride) {
+        if (p.cu_q != nullptr) return launch_prefill_d64<T, kPpVarlen, false>(p, st);
+        return launch_prefill_d64<T, kPpDense, false>(p, st);
+      }
     }
+    return launch_prefill_cfg<T, D, 4, 64, true, 2>(p, st);
   } else {
     return launch_prefill_cfg<T, D, 4, 64, GEN, 2>(p, st);
   }
@@ -243,10 +250,10 @@ hipError_t launch_fwd_d(const FwdParams& p, hipStream_t st) {
     // per key on the general one.
     if (p.block_table != nullptr) {
       if constexpr (D == 128 && !GEN) {
-        if (pp_pages(p, D)) return launch_prefill_pp<T, D, kPpVarlen, true>(p, st);
+        if (pp_pages(p, D) && row_strides_fit(p)) return launch_prefill_pp<T, D, kPpVarlen, true>(p, st);
       }
       if constexpr (D == 64 && !GEN) {
-        if (pp_pages(p, D)) return launch_prefill_d64<T, kPpVarlen, true>(p, st);
+        if (pp_pages(p, D) && row_strides_fit(p)) return launch_prefill_d64<T, kPpVarlen, true>(p, st);
       }
       using C = PrefillCfg<D>;
       return launch_fwd_cfg<T, D, C::NW, C::BN, MODE, GEN>(p, p.seqlen_q, p.heads_q * p.batch, st);
