@@ -830,18 +830,18 @@ def _varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, dro
                                             max_seqlen_k, dropout_p, softmax_scale, causal,
                                             window_size, softcap, alibi)
     plain = not (paged or seqused_q is not None or seqused_k is not None)
-    if plain and not ask_alibi and chk.ranges_only():
+    if plain and not ask_alibi and dropout_p == 0.0 and chk.ranges_only():
         # Nothing below depends on a checked value: the launch goes out first,
         # guarded by the checks' device flags, and the host waits for the checks
-        # (the one synchronization of this call) while it runs.
-        seed = new_dropout_seed() if dropout_p > 0.0 else 0
+        # (the one synchronization of this call) while it runs.  (A dropout seed
+        # is drawn only once the checks have passed: a rejected call leaves the
+        # generator alone.)
         scale = 1.0 / math.sqrt(q.shape[-1]) if softmax_scale is None else softmax_scale
         result = []
         chk.flush(lambda guard: result.append(varlen_attention(
             q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, softmax_scale=scale,
             causal=causal, window_left=window_size[0], window_right=window_size[1],
-            softcap=softcap, alibi=alibi, dropout_p=dropout_p, dropout_seed=seed, guard=guard,
-            packed=packed, covered=True)), guarded=True)
+            softcap=softcap, alibi=alibi, guard=guard, packed=packed, covered=True)), guarded=True)
         return result[0]
     values = chk.flush()   # the one host synchronization of this call
     seed = new_dropout_seed() if dropout_p > 0.0 else 0

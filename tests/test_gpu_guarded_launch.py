@@ -162,3 +162,18 @@ def test_update_writes_lengths_without_work():
         guard = torch.tensor([0, flag], dtype=torch.int32, device=DEV)
         _native.kvcache_update(None, None, kc, kc, lens, None, None, None, 16, None, None, True, q, None, out, guard)
         assert out.tolist() == ([-7] * 3 if flag else [5, 0, 16])
+
+
+def test_rejected_dropout_call_leaves_the_generator():
+    from flash_attn_triton import flash_attn_varlen_func
+    q = randn((20, 2, D), 41).to(DEV)
+    good, bad = (torch.tensor(c, dtype=torch.int32, device=DEV) for c in ([0, 7, 20], [0, 7, 19]))
+    torch.manual_seed(5)
+    state = torch.get_rng_state()
+    with pytest.raises(ValueError, match="cover"):
+        flash_attn_varlen_func(q, q, q, bad, bad, 13, 13, dropout_p=0.5)
+    assert torch.equal(torch.get_rng_state(), state)
+    first = flash_attn_varlen_func(q, q, q, good, good, 13, 13, dropout_p=0.5)
+    assert not torch.equal(torch.get_rng_state(), state)   # one draw per call that runs
+    torch.manual_seed(5)
+    assert torch.equal(flash_attn_varlen_func(q, q, q, good, good, 13, 13, dropout_p=0.5), first)
