@@ -163,7 +163,6 @@ void fwd_kernel(const FwdParams p) {
   const uint16_t* vg = static_cast<const uint16_t*>(p.v);
   uint16_t* og = static_cast<uint16_t*>(p.o);
 
-  if (MODE == kModePrefill && guard_failed(p)) return;
   int Sq, Sk;
   int64_t qoff = 0;
   int64_t q_base, o_base, lse_base;
@@ -173,6 +172,7 @@ void fwd_kernel(const FwdParams p) {
   if (MODE == kModePrefill) {
     kvh = hh / p.group;
     if (p.cu_q != nullptr) {
+      if (guard_failed(p)) return;
       const int qs = p.cu_q[b], ks = p.cu_k[b];
       Sq = p.cu_q[b + 1] - qs;
       Sk = p.cu_k[b + 1] - ks;

@@ -47,11 +47,11 @@ hipError_t launch_fwd_cfg(FwdParams p, int rows_for_grid, int outer_blocks, hipS
 // Measured on MI355X at B4 H32 S4096 D128: the masked choice is ahead on
 // causal and varlen (less work past the diagonal / sequence end), the
 // unmasked one on non-causal.
-template <class T, int D, int NW, int BN, bool GEN, int WPE, bool BIAS = false, int KS = 0>
-hipError_t launch_prefill_cfg(FwdParams p, hipStream_t st) {
+template <class T, int D, int NW, int BN, bool GEN, int WPE, bool BIAS, int KS, bool VARLEN>
+hipError_t launch_prefill_form(FwdParams p, hipStream_t st) {
   using Tile = PrefillTile<D, NW, BN>;
   constexpr int kLds = prefill_lds_bytes<D, NW, BN, KS>();
-  auto kern = prefill_kernel<T, D, NW, BN, GEN, WPE, BIAS, KS>;
+  auto kern = prefill_kernel<T, D, NW, BN, GEN, WPE, BIAS, KS, VARLEN>;
   static std::atomic<uint64_t> lds_devices{0};
   if (hipError_t e = set_lds_limit(lds_devices, kern, kLds); e != hipSuccess) return e;
   p.n_mblocks = (p.seqlen_q + Tile::BM - 1) / Tile::BM;
@@ -61,6 +61,12 @@ hipError_t launch_prefill_cfg(FwdParams p, hipStream_t st) {
   p.total_blocks = (int)total;
   hipLaunchKernelGGL(kern, dim3((unsigned)total), dim3(Tile::NT), kLds, st, p);
   return hipGetLastError();
+}
+
+template <class T, int D, int NW, int BN, bool GEN, int WPE, int KS = 0>
+hipError_t launch_prefill_cfg(const FwdParams& p, hipStream_t st) {
+  if (p.cu_q != nullptr) return launch_prefill_form<T, D, NW, BN, GEN, WPE, false, KS, true>(p, st);
+  return launch_prefill_form<T, D, NW, BN, GEN, WPE, false, KS, false>(p, st);
 }
 
 // Ping-pong prefill (fa_prefill_pp.h): 8 waves, 256 rows per workgroup.
@@ -197,8 +203,8 @@ hipError_t launch_prefill(const FwdParams& p, hipStream_t st) {
     // attn_bias (the materialized-probabilities option): 2 waves per SIMD
     // leave room for the bias loads.
     if (p.bias != nullptr) {
-      if constexpr (D == 256) return launch_prefill_cfg<T, D, 8, 32, true, 2, true>(p, st);
-      else return launch_prefill_cfg<T, D, 4, (D == 128 ? 32 : 64), true, 2, true>(p, st);
+      if constexpr (D == 256) return launch_prefill_form<T, D, 8, 32, true, 2, true, 0, false>(p, st);
+      else return launch_prefill_form<T, D, 4, (D == 128 ? 32 : 64), true, 2, true, 0, false>(p, st);
     }
   }
   const bool masked = p.causal || p.window_left >= 0 || p.window_right >= 0 || p.cu_q != nullptr;
@@ -225,8 +231,8 @@ hipError_t launch_prefill(const FwdParams& p, hipStream_t st) {
       // (40 KiB: four workgroups per CU).  Measured there on one MI355X:
       // 884 us against 927 us with the tiles staged through VGPRs; the 4-wave
       // form with 5 + 4 stages measured 927 us.
-      if (masked) return launch_prefill_cfg<T, D, 2, 32, true, 2, false, 3>(p, st);
-      return launch_prefill_cfg<T, D, 8, 64, true, 2>(p, st);
+      if (masked) return launch_prefill_cfg<T, D, 2, 32, true, 2, 3>(p, st);
+      return launch_prefill_form<T, D, 8, 64, true, 2, false, 0, false>(p, st);
     }
   } else if constexpr (D == 256) {
     return launch_prefill_cfg<T, D, 8, 32, GEN, 2>(p, st);

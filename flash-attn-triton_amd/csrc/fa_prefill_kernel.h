@@ -85,10 +85,17 @@ constexpr int prefill_lds_bytes() {
 // BIAS: the additive fp32 attn_bias is read in the score epilogue (GENERIC
 // only).  It is a separate instantiation because its per-score loads raise
 // register pressure past the budget of the 3-waves-per-SIMD tiles.
-template <class T, int D, int NW, int BN, bool GENERIC, int WPE, bool BIAS = false, int KS = 0>
+// VARLEN: cu_seqlens addressing, also an instantiation of its own.  With the
+// guard and the ranking of the sequences in the dense kernel its key loop is
+// the same instruction for instruction, but ran 5-7 % slower at head dim 32
+// where that code had moved it (fp16 causal, one MI355X: B4 S1024 H8 20.9 us
+// with it and 19.3 without, B2 S4096 H16 115 and 109 us).
+template <class T, int D, int NW, int BN, bool GENERIC, int WPE, bool BIAS = false, int KS = 0,
+          bool VARLEN = false>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
 void prefill_kernel(const FwdParams p) {
   static_assert(GENERIC || !BIAS, "the bias is applied by the generic epilogue");
+  static_assert(!VARLEN || !BIAS, "attn_bias: dense only");
   constexpr bool kDma = KS > 0;
   static_assert(!kDma || (D == 128 && BN == 32 && !BIAS && KS >= 3),
                 "the LDS-DMA ring is laid out for head dim 128 and 32-key tiles");
@@ -122,17 +129,17 @@ void prefill_kernel(const FwdParams p) {
   // first): the wider span of the ping-pong kernels doubled the HBM reads at
   // the varlen configuration.
   int mb, id;
-  if (p.cu_q == nullptr ||
+  if (!VARLEN ||
       !work_item_kv_rr(blockIdx.x, p.total_blocks, p.n_mblocks, p.group, p.heavy_first != 0, 1, mb, id))
     work_item(blockIdx.x, p.total_blocks, p.n_mblocks, p.heavy_first != 0, 1, mb, id);
-  if (guard_failed(p)) return;
   const int hh = id % p.heads_q;
   int b = id / p.heads_q;
   const int kvh = hh / p.group;
 
   int Sq, Sk;
   int64_t q_base, o_base, lse_base, k_base, v_base;
-  if (p.cu_q != nullptr) {
+  if constexpr (VARLEN) {
+    if (guard_failed(p)) return;
     const VarlenSeq sq = nth_longest(p.cu_q, p.cu_k, p.batch, b);
     const int qs = sq.qs, ks = sq.ks;
     b = sq.b;
