@@ -881,11 +881,18 @@ def _varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, dro
                             dropout_p=dropout_p, dropout_seed=seed, packed=packed, covered=True)
 
 
+_VARLEN_TENSORS = {"q", "k", "v", "cu_seqlens_q", "cu_seqlens_k", "max_seqlen_q", "max_seqlen_k"}
+
+
 def _varlen_options(window_size=(-1, -1), softcap=0.0, alibi_slopes=None, deterministic=False,
                     return_attn_probs=False, block_table=None, seqused_q=None, seqused_k=None,
                     **kwargs):
     """The options of ``flash_attn_varlen_func`` that ``_varlen`` takes; the
-    others are accepted and unused, as there."""
+    others are accepted and unused, as there, except the arguments that the
+    packed forms fill in themselves."""
+    for name in kwargs:
+        if name in _VARLEN_TENSORS:
+            raise TypeError(f"flash_attn_varlen_func() got multiple values for argument {name!r}")
     return dict(window_size=window_size, softcap=softcap, alibi_slopes=alibi_slopes,
                 return_attn_probs=return_attn_probs, block_table=block_table, seqused_q=seqused_q,
                 seqused_k=seqused_k)

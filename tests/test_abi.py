@@ -141,6 +141,18 @@ def test_python_api_validation_on_cpu():
                                4, 4)
 
 
+@pytest.mark.parametrize("name", ["q", "k", "v", "cu_seqlens_q", "cu_seqlens_k", "max_seqlen_q", "max_seqlen_k"])
+def test_packed_varlen_refuses_arguments_it_fills_in(name):
+    from flash_attn_triton import flash_attn_varlen_kvpacked_func, flash_attn_varlen_qkvpacked_func
+    x, cu = torch.zeros(4, 3, 2, 64, dtype=torch.float16), torch.tensor([0, 4], dtype=torch.int32)
+    with pytest.raises(TypeError, match=f"multiple values for argument '{name}'"):
+        flash_attn_varlen_qkvpacked_func(x, cu, 4, **{name: 3})
+    with pytest.raises(TypeError, match=f"multiple values for argument '{name}'"):
+        flash_attn_varlen_kvpacked_func(x[:, 0], x[:, 1:], cu, cu, 4, 4, **{name: 3})
+    with pytest.raises(ValueError, match="CUDA"):   # names it does not know are accepted and unused
+        flash_attn_varlen_qkvpacked_func(x, cu, 4, unknown=3)
+
+
 def test_deferred_checks_keep_the_reference_order():
     """Device-side checks are read with one synchronization, but a later host
     check never overtakes an earlier failing device check."""
