@@ -38,16 +38,40 @@ def test_dense(sq, sk, causal, window, head_dim, hq, hk, dtype):
     _check(got, ref[:3], dtype)
 
 
-# 300 workgroups of 128 keys is the last count of the two-pair form (causal): both sides of it, and group counts that
-# do and do not fill the spans.
-@pytest.mark.parametrize("batch,heads", [(1, 3), (20, 5), (60, 5), (61, 5), (25, 8)])
-def test_causal_counts(batch, heads):
+def _counts(batch, heads, causal):
     from flash_attn_triton import flash_attn_func
     s, d = 140, 64
     q, k, v, dout = (randn((batch, s, heads, d), i) for i in (11, 12, 13, 14))
     leaves = [t.to(DEV).requires_grad_() for t in (q, k, v)]
-    got = torch.autograd.grad(flash_attn_func(*leaves, causal=True), leaves, dout.to(DEV))
-    ref = ora.attention_backward(to_np(q), to_np(k), to_np(v), to_np(dout), causal=True)
+    got = torch.autograd.grad(flash_attn_func(*leaves, causal=causal), leaves, dout.to(DEV))
+    ref = ora.attention_backward(to_np(q), to_np(k), to_np(v), to_np(dout), causal=causal)
+    _check(got, ref[:3], torch.float16)
+
+
+# 300 workgroups of 128 keys is the last count of the two-pair form (causal), 150 without a mask: both sides of them (140
+# keys are two workgroups a head, so 300 and 302, 150 and 152), and group counts that do and do not fill the spans.
+@pytest.mark.parametrize("batch,heads", [(1, 3), (20, 5), (30, 5), (151, 1), (60, 5), (61, 5), (25, 8)])
+def test_causal_counts(batch, heads):
+    _counts(batch, heads, True)
+
+
+@pytest.mark.parametrize("batch,heads", [(15, 5), (19, 4)])
+def test_full_counts(batch, heads):
+    _counts(batch, heads, False)
+
+
+# A varlen launch counts by its packed keys: 10 sequences of 1910 keys in all are 14 + 5 workgroups a head (the grid,
+# sized for the longest, has 130): 285 and 304 (causal), 133 and 152 with 15, 16, 7 and 8 heads.
+@pytest.mark.parametrize("heads,causal", [(15, True), (16, True), (7, False), (8, False)])
+def test_varlen_workgroup_counts(heads, causal):
+    from flash_attn_triton import flash_attn_varlen_func
+    lengths, d = [30] * 4 + [1640] + [30] * 5, 64
+    cu = torch.tensor(np.concatenate([[0], np.cumsum(lengths)]), dtype=torch.int32)
+    q, k, v, dout = (randn((int(cu[-1]), heads, d), i) for i in (31, 32, 33, 34))
+    leaves = [t.to(DEV).requires_grad_() for t in (q, k, v)]
+    out = flash_attn_varlen_func(*leaves, cu.to(DEV), cu.to(DEV), max(lengths), max(lengths), causal=causal)
+    got = torch.autograd.grad(out, leaves, dout.to(DEV))
+    ref = ora.attention_varlen_backward(to_np(q), to_np(k), to_np(v), to_np(dout), cu.numpy(), cu.numpy(), None, causal)
     _check(got, ref[:3], torch.float16)
 
 
