@@ -42,14 +42,14 @@ def _decode(words: List[int], dtype: torch.dtype):
 _SIDE_STREAMS: dict = {}
 
 
-def _side_stream(device: torch.device) -> "torch.cuda.Stream":
-    """A second stream per device (default priority) for argument checks."""
+def _side_stream(device: torch.device):
+    """A second stream per device (default priority) for argument checks, and
+    an event to mark their end with (nothing waits for it)."""
     key = device.index if device.index is not None else torch.cuda.current_device()
-    st = _SIDE_STREAMS.get(key)
-    if st is None:
-        st = torch.cuda.Stream(device=key)
-        _SIDE_STREAMS[key] = st
-    return st
+    pair = _SIDE_STREAMS.get(key)
+    if pair is None:
+        pair = _SIDE_STREAMS[key] = (torch.cuda.Stream(device=key), torch.cuda.Event())
+    return pair
 
 
 def _as_int(t: torch.Tensor) -> torch.Tensor:
@@ -164,7 +164,7 @@ class Deferred:
         ranged = [i for i, it in enumerate(items) if it[0] in ("range", "minmax")]
         on_dev = [i for i in ranged if items[i][4][0].is_cuda]
         results = {i: _host_minmax(*items[i][4]) for i in ranged if not items[i][4][0].is_cuda}
-        done = host_rng = guard = handle = None
+        done = host_rng = guard = handle = marker = None
         jobs, job_of = [], {}
         if on_dev:
             seen = {}
@@ -185,7 +185,7 @@ class Deferred:
             device = jobs[0][0].device
             stream = torch.cuda.current_stream(device)
             if self._side:
-                side = _side_stream(device)
+                side, marker = _side_stream(device)
                 side.wait_stream(stream)
                 stream = side
             handle = stream.cuda_stream
@@ -225,6 +225,13 @@ class Deferred:
                 launch(guard) if guarded else launch()
             except Exception as exc:   # a failing check goes first
                 failed = exc
+        if marker is not None:
+            # Without a marker behind the checks the attention kernel beside them
+            # runs 1-3 % slower: one token of 32 (64) sequences of 7000 keys, 8 KV
+            # heads of 128, bf16, MI355X: 157.9 (294.5) us a call, 153.4 (289.5)
+            # with it.  Recorded here, its 3 us of host time pass while the
+            # checks run.
+            marker.record(stream)
         # Every tensor checked on the device is referenced by `items` until this
         # wait: none returns to the caching allocator (whose next user could
         # overwrite it on the current stream) while a check reads it, and the
