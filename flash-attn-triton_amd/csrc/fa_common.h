@@ -209,8 +209,13 @@ __host__ __device__ inline bool work_item_kv_rr(int L, int total, int n_mblocks,
 // sequence.  Measured on one MI355X, causal, forward / backward, before and
 // after (with the spans below): 8 sequences of 150 to 1999 tokens, Hq16 Hk4
 // D128 bf16, 97.5 / 351 -> 79.6 / 292 us; 20 of 300 and 2000, H16 D64 fp16, 75.6
-// / 294 -> 69.9 / 262 us; 24 of 128 to 2428, H16 D128 bf16, 307 / 983 -> 306 /
-// 995 us.
+// / 294 -> 69.9 / 262 us.  The order alone, against batch order with the same
+// spans: 32 of 128 to 4096, H16 D64 fp16, 706 / 2960 -> 630 / 2370 us; 24 of
+// 128 to 2428, H16 D128 bf16, 372 / 1090 -> 368 / 1105 us; what it costs where
+// every sequence is short: 64 of 512, H16 D64, 79 / 346 -> 85 / 371 us, 300 of
+// 64 to 512, H16 D128, 513 / 1380 -> 538 / 1443 us.  (A search for the r-th
+// length over ballots takes fewer instructions there, but moved these launches
+// by 5 % either way with where the code landed.)
 struct VarlenSeq {
   int b, qs, Sq, ks, Sk;
 };

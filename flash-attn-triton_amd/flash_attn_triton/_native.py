@@ -383,7 +383,8 @@ def check_ranges(arrays, minmax, diff=None) -> None:
     """min / max of each ``a`` (+ ``b``) of ``arrays`` = [(a, b or None), ...]
     (contiguous int32 / int64 device tensors, at most MAX_RANGE_CHECKS) into
     ``minmax`` (int64, 2 per array: pinned host or device memory), in one
-    launch on the current stream (fa_check_ranges).  ``diff[i]`` true: the
+    launch on the current stream (fa_check_ranges; the calls of this package
+    queue theirs with check_bounds).  ``diff[i]`` true: the
     adjacent differences of ``a`` instead (``b`` must be None)."""
     lib = load()
     n = len(arrays)

@@ -734,7 +734,7 @@ def _varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, dro
     # With seqused_* the reference re-derives that side's cu_seqlens from the
     # used counts (:563, :581), so its start/order/size checks always pass.
     # Range checks on cu_seqlens slices and on its adjacent differences (the
-    # sequence lengths): all of them reduce in one fa_check_ranges launch.
+    # sequence lengths): all of them reduce in one fa_check_bounds launch.
     cu_q_first, cu_k_first = cu_seqlens_q[:1], cu_seqlens_k[:1]
     cu_q_last, cu_k_last = cu_seqlens_q[-1:], cu_seqlens_k[-1:]
     if seqused_q is None:

@@ -1,10 +1,11 @@
-"""The decode call's argument checks on the GPU (fa_check_ranges).
+"""The decode call's argument checks on the GPU (fa_check_bounds), and the
+reduction by itself (fa_check_ranges).
 
 A plain decode call (no append, rotary or ALiBi) launches before it waits
 for its checks: the range checks of the block table, cache_seqlens,
-cache_batch_idx and cache_leftpad reduce in one fa_check_ranges launch on a
-second stream into pinned host memory, and the reference's ValueError is
-raised after the launch (flash_attn_interface.py:428-453).  The kernels
+cache_batch_idx and cache_leftpad reduce in one fa_check_bounds launch (on a
+second stream where the attention outlasts the host's work) into pinned host
+memory, and the reference's ValueError is raised after the launch (flash_attn_interface.py:428-453).  The kernels
 clamp cache lengths and left pads to the cache, so the failing cases here
 feed only out-of-range lengths / pads (never page indices or cache rows
 outside the cache).
