@@ -217,8 +217,8 @@ class Deferred:
             else:
                 words = packed.tolist()
         failed = None
-        # (`results` holds the host tensors' ranges so far.)
-        if guarded and any(_outside(items[i], r) for i, r in results.items()):
+        # (`results` holds the host tensors' ranges so far, mostly none.)
+        if guarded and results and any(_outside(items[i], r) for i, r in results.items()):
             launch = None
         if launch is not None:
             try:
@@ -253,9 +253,10 @@ class Deferred:
             scalars_dec.append(_decode(words[pos:pos + n], dt))
             pos += n
         values, k = [], 0
-        for i, (kind, exc, _, _, _) in enumerate(items):
+        for i, (kind, exc, lo, hi, _) in enumerate(items):
             if kind == "range":
-                if _outside(items[i], results[i]):
+                mn, mx = results[i]
+                if (lo is not None and mn < lo) or (hi is not None and mx > hi):
                     raise exc
             elif kind == "minmax":
                 values.append(results[i])
